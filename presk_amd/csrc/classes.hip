@@ -138,7 +138,9 @@ struct GemmPlan : ClassPlan {
     std::string order() const override {
         // 16-bit storage: 32x32x16 MFMAs (k in steps of 16) on every tile but
         // the 128 x 96 one (16x16x32, steps of 32)
-        std::string o = storage == kF32 ? "mfma-f32-k4" : g.bm == 256 || g.bn != 96 ? "mfma-k16" : "mfma-k32";
+        // f32 storage: 16x16x4 MFMAs, or products of operands split in three
+        // bf16 parts (32x32x16)
+        std::string o = storage == kF32 ? g.split3 ? "mfma-f32x3-k16" : "mfma-f32-k4" : g.bm == 256 || g.bn != 96 ? "mfma-k16" : "mfma-k32";
         if (g.splits > 1) o += "-split" + std::to_string(g.splits);
         return o;
     }
@@ -322,11 +324,70 @@ void apply_override(GemmArgs& g) {
     }
 }
 
-void plan_tiles(GemmArgs& g) {
+// f32 operands split in three bf16 parts on the bf16 matrix cores
+// (gemm_split.hip): 128-row tiles of 192 or 128 columns by eight waves (one
+// workgroup a CU), 128 or 64 columns by four (two a CU).  A CU's time over
+// the workgroups it is dealt is modelled as its columns over an efficiency
+// measured at full occupancy -- 192 columns 1 (16384 x 384 x 1536 109 us),
+// 128 by eight waves 0.92 (4096 x 1024 x 1024 51 us), by four 1 in pairs
+// (16384 x 1536 x 384 122 us, where the pair's stores overlap) and 0.77
+// alone (61 us), 64 columns 0.85 and 0.65 -- the earlier on a tie.  A long K
+// over few tiles is split as the f32 tiles' is: as many ranges as fill one
+// round of the CUs, each of at least four 32-deep blocks, or of twelve from
+// 64 tiles on (16384 x 128 x 384 as 128 tiles split in two measured 24 us
+// against 21 unsplit: the partials' round trip).
+void plan_split3(GemmArgs& g) {
+    g.split3 = true;
+    g.bm = 128;
+    g.eight = false;
+    g.stream = false;
+    g.splits = 1;
+    g.k_per_split = g.K;
+    g.tiles_m = (int)((g.M + 127) / 128);
+    const long long rows = (long long)g.tiles_m * g.batch, nkb = (g.K + 31) / 32;
+    const long long t128 = rows * ((g.N + 127) / 128);
+    if (g.batch == 1 && t128 < 256 && nkb >= 8) {
+        long long s = 256 / t128;
+        const long long least = t128 < 64 ? 4 : 12;
+        if (s > nkb / least) s = nkb / least;
+        if (s > 64) s = 64;
+        if (s > 1) {
+            g.bn = 128;
+            g.eight = true;
+            g.tiles_n = (int)((g.N + 127) / 128);
+            g.splits = (int)s;
+            g.k_per_split = (nkb + s - 1) / s * 32;
+            return;
+        }
+    }
+    struct Shape { int bn; bool eight; double pair, alone; };
+    static const Shape shapes[4] = {{128, false, 1.0, 0.77}, {192, true, 1.0, 1.0}, {128, true, 0.92, 0.92}, {64, false, 0.85, 0.65}};
+    double best = -1;
+    for (const Shape& h : shapes) {
+        const long long t = rows * ((g.N + h.bn - 1) / h.bn), r = (t + 255) / 256;
+        const double cost = h.bn * ((double)(r / 2 * 2) / h.pair + (double)(r % 2) / h.alone);
+        if (best < 0 || cost < best) {
+            best = cost;
+            g.bn = h.bn;
+            g.eight = h.eight;
+        }
+    }
+    g.tiles_n = (int)((g.N + g.bn - 1) / g.bn);
+}
+
+void plan_tiles(GemmArgs& g, bool widened) {
+    g.split3 = false;
     g.bm = 128;
     g.eight = false;
     g.stream = true;
     g.tiles_m = (int)((g.M + gemm_tile_m() - 1) / gemm_tile_m());
+    // (operands widened from other types and named tiles keep the f32 MFMAs)
+    TileOverride named;
+    std::string ignored;
+    if (!widened && gemm_split_fits(g) && (!tile_override(&named, &ignored) || named.bm == 0)) {
+        plan_split3(g);
+        return;
+    }
     long long best = -1;
     if (g.storage == kF32) {
         // tile columns: 128, 96 or 64, whichever finishes first when the
@@ -743,7 +804,7 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k) {
     g.a_kcontig = g.sa_k == 1;
     g.b_kcontig = g.sb_k == 1;
     if (g.M <= 0 || g.N <= 0 || g.K <= 0) return nullptr;
-    plan_tiles(g);
+    plan_tiles(g, wide);
     if (g.batch > 65535 || g.splits > 65535) return nullptr;
     // 32-bit element offsets inside one batch entry
     const double lim = 2147483647.0;

@@ -28,8 +28,11 @@
 // k-blocks take four-wave tiles and the same MFMAs from register-staged
 // operands; 128 x 96 tiles take the 16x16 MFMAs below.
 //
-// f32 storage, whole 32-deep k-blocks and strides of whole vectors: eight-wave
-// tiles too (F32Loader), 256 x 128 and 256 x 96 three k-blocks deep, 128 x
+// f32 storage: products of operands split in three bf16 parts where that is
+// faster (gemm_split.hip; order "mfma-f32x3-k16"); what is described here for
+// f32 are the 16x16x4 tiles, which short K, few rows or columns and operands
+// widened from e8m15 or integer weights take.  Whole 32-deep k-blocks and
+// strides of whole vectors: eight-wave tiles too (F32Loader), 256 x 128 and 256 x 96 three k-blocks deep, 128 x
 // 128 four deep (split weight gradients among them) and 128 x 96 two deep
 // (two workgroups a CU), each wave's
 // 16x16x4 MFMAs taking the operands' roles exchanged so that its sums leave
@@ -1330,6 +1333,12 @@ hipError_t launch_typed(const GemmArgs& g, hipStream_t stream) {
     const bool fast = g.a_vec && g.b_vec;
     hipError_t e;
     if (stream_fits(g)) return stream_launch<ST>(g, stream);
+    if (ST == kF32 && g.split3) {
+        e = gemm_split_launch(g, stream);
+        if (e != hipSuccess || g.splits <= 1) return e;
+        split_reduce_kernel<ST><<<(unsigned)((g.M * g.N + 255) / 256), 256, 0, stream>>>(g);
+        return hipGetLastError();
+    }
     if constexpr (ST == kF32) {
     if (g.bm == 256 || g.eight) {
         // 256 x 128 or 256 x 96 tiles of eight waves (4 x 2 waves of 64 x 64

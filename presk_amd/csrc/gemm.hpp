@@ -31,10 +31,16 @@ struct GemmArgs {
     int bm;                         // tile rows: 128, or 256 (eight-wave tiles)
     int bn;                         // tile columns: 256, 128, 96 or 64
     bool eight;                     // 128-row tiles of eight waves: 128 x 128, or 128 x 96 in f32 (256-row tiles always have eight)
+    bool split3;                    // f32 on the bf16 matrix cores (gemm_split.hip): 128 rows, 192, 128 (eight or four waves) or 64 columns
     bool stream;                    // K of at most two k-blocks may stream B's tiles across a kept A panel
 };
 
 hipError_t gemm_launch(const GemmArgs& g, hipStream_t stream);
+
+// f32 products as six bf16 products of operands split in three (gemm_split.hip);
+// the split-K partials' reduction is the caller's
+bool gemm_split_fits(const GemmArgs& g);
+hipError_t gemm_split_launch(const GemmArgs& g, hipStream_t stream);
 
 // e8m15 contractions (the f32 kernel on exact widenings): an e8m15 code is
 // the top 24 bits of its f32, so the n codes at src widen to dst exactly
