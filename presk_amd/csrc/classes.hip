@@ -7,12 +7,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <functional>
 #include <map>
 #include <mutex>
+#include <set>
 
 #include "devfmt.hpp"
 #include "executor.hpp"
@@ -107,6 +109,213 @@ bool product_pattern(const Kernel& k, std::vector<int>* vars0, std::vector<int>*
     return vars(load0, vars0) && vars(load1, vars1);
 }
 
+// Whether the nest sums each output's products in index order into one
+// accumulator from zero and stores it (with an epilogue, reads it back and
+// adds the bias, in f32 before the store): every layout point of a contraction does, a nest under
+// a realization's `interleaved` or `chunked` order does not.  The summed
+// loops stand inside the output's, in the order of operand 0's axes, around
+// nothing but `x = %0[..]` and `acc = acc + x * %1[..]`, the accumulators set
+// to zero just outside them.
+bool sequential_sum(const Kernel& k) {
+    std::set<int> out_vars, accs, vaccs;
+    std::function<void(const Expr*, std::set<int>&)> ivs = [&](const Expr* e, std::set<int>& v) {
+        if (e->kind == Expr::Iv) v.insert(e->id);
+        for (auto c : e->kids) ivs(c, v);
+    };
+    std::function<void(const std::vector<const Stmt*>&)> outs = [&](const std::vector<const Stmt*>& body) {
+        for (auto s : body) {
+            for (auto e : s->index) ivs(e, out_vars);
+            outs(s->body);
+        }
+    };
+    outs(k.body);
+    std::vector<int> summed;          // the summed loops, outermost first
+    int stores = 0, terms = 0, biased = 0, read_back = 0;
+    bool ok = true;
+    auto is_load = [&](const Expr* e, int b) {
+        if ((e->kind != Expr::Load && e->kind != Expr::VLoad) || e->id != b) return false;
+        // the summed loops index their axes by themselves
+        for (auto c : e->kids) {
+            std::set<int> v;
+            ivs(c, v);
+            for (int u : v)
+                if (!out_vars.count(u) && c->kind != Expr::Iv) return false;
+        }
+        return true;
+    };
+    auto plain = [](const Expr* e) { return e->kind == Expr::Splat ? e->kids[0] : e; };
+    std::function<void(const std::vector<const Stmt*>&, bool)> walk = [&](const std::vector<const Stmt*>& body, bool inside) {
+        int x = -1;                   // the scalar holding %0's element
+        for (size_t i = 0; ok && i < body.size(); ++i) {
+            const Stmt* s = body[i];
+            if (s->kind == Stmt::For) {
+                const bool sum = !out_vars.count(s->var);
+                if (inside && !sum) ok = false;                 // an output loop inside a summed one
+                if (sum) {
+                    // one chain of summed loops in the nest
+                    if (!inside && !summed.empty()) ok = false;
+                    if (inside && body.size() != 1) ok = false;
+                    summed.push_back(s->var);
+                }
+                walk(s->body, inside || sum);
+            } else if (s->kind == Stmt::Set || s->kind == Stmt::VSet) {
+                const bool vec = s->kind == Stmt::VSet;
+                std::set<int>& as = vec ? vaccs : accs;
+                const Expr* v = plain(s->value);
+                if (!inside && !summed.empty()) {
+                    // the epilogue in f32: the bias added to the sum before
+                    // its store (once an accumulator)
+                    const Expr* e = s->value;
+                    const bool add = (e->kind == Expr::Bin || e->kind == Expr::VBin) && e->op == Op::Add;
+                    if (!add || k.dtype != Ty::F32 || k.inputs.size() != 3 || !as.count(s->var) ||
+                        e->kids[0]->kind != (vec ? Expr::Vv : Expr::Sv) || e->kids[0]->id != s->var) { ok = false; break; }
+                    const Expr* b = plain(e->kids[1]);
+                    if ((b->kind != Expr::Load && b->kind != Expr::VLoad) || b->id != 2) ok = false;
+                    ++biased;
+                    continue;
+                }
+                if (!inside) {
+                    if (v->kind != Expr::Num || v->num != 0 || std::signbit(v->num)) ok = false;
+                    as.insert(s->var);
+                    continue;
+                }
+                if (!vec && is_load(s->value, 0) && !accs.count(s->var)) {
+                    x = s->var;
+                    continue;
+                }
+                const Expr* e = s->value;
+                if ((e->kind != Expr::Bin && e->kind != Expr::VBin) || e->op != Op::Add || !as.count(s->var)) { ok = false; break; }
+                const Expr *a = e->kids[0], *m = e->kids[1];
+                if (a->kind != (vec ? Expr::Vv : Expr::Sv) || a->id != s->var) { ok = false; break; }
+                if ((m->kind != Expr::Bin && m->kind != Expr::VBin) || m->op != Op::Mul || !is_load(m->kids[1], 1)) { ok = false; break; }
+                const Expr* l = plain(m->kids[0]);
+                // the generic `ein` term (1 * x0) * x1: 1 * x0 is x0 exactly
+                if (l->kind == Expr::Bin && l->op == Op::Mul && l->kids[0]->kind == Expr::Num && l->kids[0]->num == 1) l = l->kids[1];
+                if (!(l->kind == Expr::Sv && l->id == x && x >= 0) && !is_load(l, 0)) { ok = false; break; }
+                ++terms;
+            } else if (s->kind == Stmt::Store || s->kind == Stmt::VStore) {
+                if (inside || summed.empty() || s->buf != k.out_buf()) { ok = false; break; }
+                const Expr* v = s->value;
+                if ((v->kind == Expr::Sv && accs.count(v->id)) || (v->kind == Expr::Vv && vaccs.count(v->id))) {
+                    ++stores;
+                    continue;
+                }
+                // the epilogue: the stored element read back, plus the bias
+                const bool add = (v->kind == Expr::Bin || v->kind == Expr::VBin) && v->op == Op::Add;
+                if (!add || k.inputs.size() != 3) { ok = false; break; }
+                const Expr *o = v->kids[0], *b = plain(v->kids[1]);
+                auto same = [&](const std::vector<const Expr*>& p, const std::vector<const Expr*>& q) {
+                    if (p.size() != q.size()) return false;
+                    for (size_t d = 0; d < p.size(); ++d)
+                        if (show_expr(*p[d]) != show_expr(*q[d])) return false;
+                    return true;
+                };
+                if ((o->kind != Expr::Load && o->kind != Expr::VLoad) || o->id != k.out_buf() || !same(o->kids, s->index) ||
+                    (b->kind != Expr::Load && b->kind != Expr::VLoad) || b->id != 2)
+                    ok = false;
+                ++read_back;
+            } else {
+                ok = false;
+            }
+        }
+    };
+    walk(k.body, false);
+    if (biased + read_back != (k.inputs.size() == 3 ? stores : 0)) return false;
+    if (!ok || summed.empty() || stores == 0 || stores != terms || (int)(accs.size() + vaccs.size()) < stores) return false;
+    // the summed loops in the order of operand 0's axes
+    std::vector<int> axes;
+    std::function<bool(const std::vector<const Stmt*>&)> first = [&](const std::vector<const Stmt*>& body) {
+        std::function<bool(const Expr*)> find = [&](const Expr* e) {
+            if ((e->kind == Expr::Load || e->kind == Expr::VLoad) && e->id == 0) {
+                for (auto c : e->kids)
+                    if (c->kind == Expr::Iv && !out_vars.count(c->id)) axes.push_back(c->id);
+                return true;
+            }
+            for (auto c : e->kids)
+                if (find(c)) return true;
+            return false;
+        };
+        for (auto s : body)
+            if ((s->value && find(s->value)) || first(s->body)) return true;
+        return false;
+    };
+    return first(k.body) && axes == summed;
+}
+
+// The row-wise layout of an f32 contraction (lower.rs:846-905): the output's
+// row set to zero, then for each k every element of it read back, its product
+// added and stored -- in f32 the stored element is the running sum, so these
+// are the same values.
+bool row_wise_sum(const Kernel& k) {
+    if (k.dtype != Ty::F32) return false;
+    std::set<int> out_vars;
+    std::function<void(const std::vector<const Stmt*>&)> outs = [&](const std::vector<const Stmt*>& body) {
+        for (auto s : body) {
+            for (auto e : s->index)
+                if (e->kind == Expr::Iv) out_vars.insert(e->id);
+            outs(s->body);
+        }
+    };
+    outs(k.body);
+    bool ok = true;
+    int zeros = 0, terms = 0, biased = 0;
+    std::vector<int> summed, axes;
+    const int64_t numel = k.output.numel();
+    auto same = [&](const std::vector<const Expr*>& p, const std::vector<const Expr*>& q) {
+        if (p.size() != q.size()) return false;
+        for (size_t d = 0; d < p.size(); ++d)
+            if (p[d]->kind != Expr::Iv || q[d]->kind != Expr::Iv || p[d]->id != q[d]->id) return false;
+        return true;
+    };
+    // elems: the output elements the enclosing output loops cover
+    std::function<void(const std::vector<const Stmt*>&, bool, int64_t, int)> walk = [&](const std::vector<const Stmt*>& body,
+                                                                                       bool inside, int64_t elems, int x) {
+        for (size_t i = 0; ok && i < body.size(); ++i) {
+            const Stmt* s = body[i];
+            if (s->kind == Stmt::For) {
+                const bool sum = !out_vars.count(s->var);
+                if (sum && !inside && !summed.empty()) ok = false;      // a second chain of sums
+                if (sum) summed.push_back(s->var);
+                walk(s->body, inside || sum, sum ? elems : elems * s->bound, x);
+            } else if (s->kind == Stmt::Set) {
+                const Expr* v = s->value;
+                if (!inside || v->kind != Expr::Load || v->id != 0 || !axes.empty()) { ok = false; break; }
+                for (auto c : v->kids) {
+                    if (c->kind != Expr::Iv) ok = false;
+                    else if (!out_vars.count(c->id)) axes.push_back(c->id);
+                }
+                x = s->var;
+            } else if (s->kind == Stmt::Store) {
+                const Expr* v = s->value;
+                if (s->buf != k.out_buf() || elems != numel) { ok = false; break; }
+                if (!inside && summed.empty()) {
+                    if (v->kind != Expr::Num || v->num != 0 || std::signbit(v->num)) ok = false;
+                    ++zeros;
+                    continue;
+                }
+                if (v->kind != Expr::Bin || v->op != Op::Add) { ok = false; break; }
+                const Expr *o = v->kids[0], *t = v->kids[1];
+                if (o->kind != Expr::Load || o->id != k.out_buf() || !same(o->kids, s->index)) { ok = false; break; }
+                if (inside) {
+                    if (t->kind != Expr::Bin || t->op != Op::Mul || t->kids[0]->kind != Expr::Sv || t->kids[0]->id != x || x < 0 ||
+                        t->kids[1]->kind != Expr::Load || t->kids[1]->id != 1)
+                        ok = false;
+                    for (auto c : t->kids[1]->kids)
+                        if (c->kind != Expr::Iv) ok = false;
+                    ++terms;
+                } else {
+                    if (t->kind != Expr::Load || t->id != 2 || k.inputs.size() != 3) ok = false;
+                    ++biased;
+                }
+            } else {
+                ok = false;
+            }
+        }
+    };
+    walk(k.body, false, 1, -1);
+    return ok && zeros == 1 && terms == 1 && biased == (k.inputs.size() == 3 ? 1 : 0) && !summed.empty() && axes == summed;
+}
+
 // ---- the contraction class ---------------------------------------------------------
 struct GemmPlan : ClassPlan {
     GemmArgs g{};          // pointers filled at launch
@@ -133,9 +342,11 @@ struct GemmPlan : ClassPlan {
     bool swapped = false;          // operand 1 is A (an `ein` whose operand 1 carries I)
     long long rows_per_iter = 0;
     long long cols_per_iter = 0;
+    bool seq = false;              // EXACT: the interpreter's sums (gemm_seq.hip)
 
-    const char* kind() const override { return "gemm"; }
+    const char* kind() const override { return seq ? "seqdot" : "gemm"; }
     std::string order() const override {
+        if (seq) return "sequential";
         // 16-bit storage: 32x32x16 MFMAs (k in steps of 16) on every tile but
         // the 128 x 96 one (16x16x32, steps of 32)
         // f32 storage: 16x16x4 MFMAs, or products of operands split in three
@@ -230,6 +441,7 @@ struct GemmPlan : ClassPlan {
             if (n_out) n_out += nsz * c_off;
             if (n_bias) n_bias += nsz * bias_off;
         }
+        if (seq) return gemm_seq_launch(a, stream);
         // the clamped 16-byte loads need whole aligned vectors along the
         // loaded axis: k when it is contiguous, else the rows
         const int vec = storage == kF32 ? 4 : 8;
@@ -565,7 +777,7 @@ void plan_tiles(GemmArgs& g, bool widened) {
     apply_override(g);
 }
 
-std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k) {
+std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
     const std::string& n = k.name;
     const bool is_dot = n == "dot" || n == "dot+add";
     const bool is_l = n == "dot_vjp_l", is_r = n == "dot_vjp_r";
@@ -804,7 +1016,21 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k) {
     g.a_kcontig = g.sa_k == 1;
     g.b_kcontig = g.sb_k == 1;
     if (g.M <= 0 || g.N <= 0 || g.K <= 0) return nullptr;
-    plan_tiles(g, wide);
+    if (seq) {
+        // the printed nest where a tile's blocks would be most of the work
+        // (512 x 128 x 128, 2^23 products, takes 7.6 us in tiles and 10.5
+        // printed; 256 x 256 x 256 12.8 and 18.4)
+        const long long lim = 1ll << 22;   // 32-bit offsets inside a tile
+        if (wide || g.sa_m >= lim || g.sa_k >= lim || g.sb_k >= lim || g.sb_n >= lim ||
+            (double)g.M * g.N * g.batch * g.K < 8388608.0 || g.M < 32 || g.N < 32 ||
+            !(sequential_sum(k) || row_wise_sum(k)))
+            return nullptr;
+        p->seq = true;
+        g.splits = 1;
+        g.k_per_split = g.K;
+    } else {
+        plan_tiles(g, wide);
+    }
     if (g.batch > 65535 || g.splits > 65535) return nullptr;
     // 32-bit element offsets inside one batch entry
     const double lim = 2147483647.0;
@@ -1097,15 +1323,14 @@ std::unique_ptr<ClassPlan> classify(const Kernel& k, int mode) {
     // integer weights (their scales in the slots after the output): in
     // FAST a contraction takes the f32 MFMA kernel on their loads, anything
     // else the generic printer's loads
-    if (k.n_quant() > 0) return mode == PRESK_HIP_FAST ? classify_gemm(k) : nullptr;
+    if (k.n_quant() > 0) return mode == PRESK_HIP_FAST ? classify_gemm(k, false) : nullptr;
     // FAST: column sums and totals in the declared chunked order
     if (mode == PRESK_HIP_FAST)
         if (auto p = classify_sum_to(k)) return p;
     // row nests: the interpreter's order (EXACT), FAST's lane tree (FAST)
     if (auto p = classify_rows(k, mode == PRESK_HIP_FAST)) return p;
     if (auto p = classify_scatter(k)) return p;
-    if (mode == PRESK_HIP_FAST)
-        if (auto p = classify_gemm(k)) return p;
+    if (auto p = classify_gemm(k, mode == PRESK_HIP_EXACT)) return p;
     return nullptr;
 }
 

@@ -42,6 +42,10 @@ hipError_t gemm_launch(const GemmArgs& g, hipStream_t stream);
 bool gemm_split_fits(const GemmArgs& g);
 hipError_t gemm_split_launch(const GemmArgs& g, hipStream_t stream);
 
+// EXACT mode: each output its products' running sum in index order, the
+// product and the sum rounded to f32 (gemm_seq.hip); no split
+hipError_t gemm_seq_launch(const GemmArgs& g, hipStream_t stream);
+
 // e8m15 contractions (the f32 kernel on exact widenings): an e8m15 code is
 // the top 24 bits of its f32, so the n codes at src widen to dst exactly
 hipError_t gemm_e8_widen(const void* src, float* dst, long long n, hipStream_t stream);
