@@ -351,7 +351,7 @@ struct GemmPlan : ClassPlan {
         // the 128 x 96 one (16x16x32, steps of 32)
         // f32 storage: 16x16x4 MFMAs, or products of operands split in three
         // bf16 parts (32x32x16)
-        std::string o = storage == kF32 ? g.split3 ? "mfma-f32x3-k16" : "mfma-f32-k4" : g.bm == 256 || g.bn != 96 ? "mfma-k16" : "mfma-k32";
+        std::string o = storage == kF32 ? g.split3 || g.b_bits ? "mfma-f32x3-k16" : "mfma-f32-k4" : g.bm == 256 || g.bn != 96 ? "mfma-k16" : "mfma-k32";
         if (g.splits > 1) o += "-split" + std::to_string(g.splits);
         return o;
     }
@@ -408,6 +408,16 @@ struct GemmPlan : ClassPlan {
             work = (char*)work + wide_bytes();
         }
         const int esz = storage == kF32 ? 4 : 2;
+        // an integer B is addressed by element (int4 two a byte)
+        if (a.b_bits) a.scales = (const float*)bufs[scale_slot[swapped ? 0 : 1]];
+        auto move_b = [&](long long elements, long long scales) {
+            if (a.b_bits) {
+                a.b_elem = elements;
+                a.scales += scales;
+            } else {
+                a.B = (const char*)a.B + elements * esz;
+            }
+        };
         // a partial range: the same tiles, k-blocks and split of K as the
         // whole call, over fewer batch entries, rows or columns -- each
         // element is summed by the same steps, so its bits do not change
@@ -416,13 +426,13 @@ struct GemmPlan : ClassPlan {
             long long c_off = 0, bias_off = 0;
             if (split_on_batch) {
                 a.A = (const char*)a.A + first * a.sa_b[0] * esz;
-                a.B = (const char*)a.B + first * a.sb_b[0] * esz;
+                move_b(first * a.sb_b[0], first * a.ss_b[0]);
                 c_off = first * a.sc_b[0];
                 a.batch = a.batch / a.bdim[0] * count;
                 a.bdim[0] = count;
             } else if (cols_per_iter > 0) {
                 const long long n0 = first * cols_per_iter;
-                a.B = (const char*)a.B + n0 * a.sb_n * esz;
+                move_b(n0 * a.sb_n, n0 * a.ss_n);
                 c_off = n0;
                 if (a.bias_kind == 1) bias_off = n0;
                 a.N = count * cols_per_iter;
@@ -587,8 +597,44 @@ void plan_split3(GemmArgs& g) {
     g.tiles_n = (int)((g.N + g.bn - 1) / g.bn);
 }
 
+// Tiles and splits of the 16-bit and integer-weight products staged through
+// registers: 32 x 128 tiles for at most 32 rows, split in k until two
+// workgroups stand on every CU (each split two 64-deep blocks or more), else
+// 128 x 128, or 128 x 64 (16-bit ragged operands) where that wastes less of
+// the last column tile, split where the tiles leave CUs idle.
+void plan_staged(GemmArgs& g) {
+    g.staged = g.b_bits == 0;
+    g.stream = g.eight = false;
+    g.splits = 1;
+    g.k_per_split = g.K;
+    const int unit = g.storage == kF32 ? 32 : 64;
+    const long long nkb = (g.K + unit - 1) / unit;
+    g.bm = g.M <= 32 ? 32 : 128;
+    g.bn = g.bm == 128 && g.b_bits == 0 && (g.N + 63) / 64 % 2 ? 64 : 128;
+    g.tiles_m = (int)((g.M + g.bm - 1) / g.bm);
+    g.tiles_n = (int)((g.N + g.bn - 1) / g.bn);
+    const long long t = (long long)g.tiles_m * g.tiles_n;
+    if (g.batch == 1 && t < 256) {
+        long long s = 512 / t;
+        // few rows: eight 64-deep blocks a split, four where that leaves CUs
+        // idle (8 x 4096 x 4096 split 8 12.0 us, 16 12.6); 128-row tiles: a
+        // K of 256, or of 1024 from 96 tiles on (1999 x 1021 x 777, 208 of
+        // them: unsplit 21.1 us, 4 ways 28; 4096 x 65 x 1021, 64: unsplit
+        // 24.2, 4 ways 21.2; int8 weights from 16, their conversion being
+        // the longer part of a block: 128 x 4096 x 4096, 32 tiles, 4 ways 22.8
+        // us, 16 ways 28.4)
+        const long long least = g.bm == 32 ? (t * (nkb / 8) >= 256 ? 8 : 4) : (t < (g.b_bits ? 16 : 96) ? 256 : 1024) / unit;
+        if (s > nkb / least) s = nkb / least;
+        if (s > 64) s = 64;
+        if (s > 1) {
+            g.splits = (int)s;
+            g.k_per_split = (nkb + s - 1) / s * unit;
+        }
+    }
+}
+
 void plan_tiles(GemmArgs& g, bool widened) {
-    g.split3 = false;
+    g.split3 = g.staged = false;
     g.bm = 128;
     g.eight = false;
     g.stream = true;
@@ -599,6 +645,17 @@ void plan_tiles(GemmArgs& g, bool widened) {
     if (!widened && gemm_split_fits(g) && (!tile_override(&named, &ignored) || named.bm == 0)) {
         plan_split3(g);
         return;
+    }
+    if (g.storage != kF32 && gemm_ragged_fits(g) && (!tile_override(&named, &ignored) || named.bm == 0)) {
+        // operands whose vectors are not whole (of eight, by their sizes and
+        // strides: the pointers are the launch's), or few rows of a long K
+        bool whole = (g.a_kcontig ? g.K : g.M) % 8 == 0 && (g.b_kcontig ? g.K : g.N) % 8 == 0 &&
+                     (g.a_kcontig ? g.sa_m : g.sa_k) % 8 == 0 && (g.b_kcontig ? g.sb_n : g.sb_k) % 8 == 0;
+        for (int d = 0; d < g.nbatch; ++d) whole = whole && g.sa_b[d] % 8 == 0 && g.sb_b[d] % 8 == 0;
+        if (!whole || (g.M <= 32 && g.a_kcontig && g.K >= 512 && g.N >= 128)) {
+            plan_staged(g);
+            return;
+        }
     }
     long long best = -1;
     if (g.storage == kF32) {
@@ -777,6 +834,27 @@ void plan_tiles(GemmArgs& g, bool widened) {
     apply_override(g);
 }
 
+// Whether the nest's integer weights are B, read as integers (gemm_quant.hip):
+// their scales constant along K and at one stride along the columns, A k
+// contiguous in its own storage.  From 32 columns (narrower is a row of a
+// tile), and to 2 048 rows: longer calls keep the widened copies' order
+// "mfma-f32-k4", which their callers rely on, and where the copies are a
+// small part of the work.
+bool integer_weights(const Kernel& k, GemmPlan& p, int own, long long scale_axis, const std::vector<long long>& batch_scales) {
+    GemmArgs& g = p.g;
+    const int b = p.swapped ? 0 : 1;
+    if (own < 0 || k.dtype == Ty::E8M15 || !ty_quant(k.inputs[b].ty) || ty_quant(k.inputs[1 - b].ty)) return false;
+    if (scale_axis < 0 || (int)batch_scales.size() != g.nbatch || g.M > 2048 || g.N < 32 || !gemm_quant_fits(g)) return false;
+    g.b_bits = k.inputs[b].ty == Ty::Q8 ? 8 : 4;
+    g.ss_n = scale_axis;
+    for (int d = 0; d < g.nbatch; ++d) g.ss_b[d] = batch_scales[d];
+    g.storage = own;
+    p.storage = own;
+    p.conv[0] = p.conv[1] = 0;
+    p.narrow = -1;
+    return true;
+}
+
 std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
     const std::string& n = k.name;
     const bool is_dot = n == "dot" || n == "dot+add";
@@ -833,6 +911,11 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
     p->n_in = (int)k.inputs.size();
     p->guarded = k.guarded();
     p->nest = parallel_outer(k);
+    // an integer B's scale strides: along the columns (-1: not constant along
+    // K), and along each batch axis
+    long long scale_axis = -1;
+    std::vector<long long> batch_scales;
+    const auto ws = ty_quant(w.ty) ? w.scale_strides() : std::vector<int64_t>();
     if (is_dot) {
         // x[outer..., I, K] . w[K, J] -> [outer..., I, J]   (Contraction::of, lower.rs:700-711)
         if (w.dims.size() != 2 || x.dims.size() < 2 || x.dims.back() != w.dims[0]) return nullptr;
@@ -842,6 +925,7 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         if (o.numel() != g.M * g.N || o.dims.back() != g.N) return nullptr;
         g.sa_m = g.K; g.sa_k = 1; g.sb_k = g.N; g.sb_n = 1; g.sc_m = g.N;
         p->rows_per_iter = x.dims.size() >= 1 ? g.M / x.dims[0] : 0;
+        if (ws.size() == 2 && ws[0] == 0) scale_axis = ws[1];
     } else if (is_l) {
         // ct[outer..., I, N] . b[J, N]^T -> [outer..., I, J]   (lower.rs:715-726)
         if (w.dims.size() != 2 || x.dims.size() < 2 || x.dims.back() != w.dims[1]) return nullptr;
@@ -851,6 +935,7 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         if (o.numel() != g.M * g.N) return nullptr;
         g.sa_m = g.K; g.sa_k = 1; g.sb_k = 1; g.sb_n = g.K; g.sc_m = g.N;
         p->rows_per_iter = g.M / x.dims[0];
+        if (ws.size() == 2 && ws[1] == 0) scale_axis = ws[0];
     } else if (is_r) {
         // a[lead..., I], ct[lead..., J] -> [I, J], summed over lead   (lower.rs:730-739)
         if (x.dims.size() < 2 || x.dims.size() != w.dims.size()) return nullptr;
@@ -956,6 +1041,12 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         // first output axis (the KernelFn split loop), which is never merged
         // into; the others collapsed where all three strides allow it
         std::vector<long long> bd, ba, bb, bc;
+        const auto wss = ty_quant(wb->ty) ? wb->scale_strides() : std::vector<int64_t>(wb->dims.size(), 0);
+        if (ty_quant(wb->ty)) {
+            scale_axis = wss[pos(vb, vj)];
+            for (int v : summed)
+                if (wss[pos(vb, v)] != 0) scale_axis = -1;
+        }
         bool first_is_batch = false;
         for (size_t q = 0; q < vo.size(); ++q) {
             const int v = vo[q];
@@ -967,13 +1058,16 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
             if (q == 0) first_is_batch = true;
             else if (n == 1) continue;
             const bool mergeable = !bd.empty() && !(first_is_batch && bd.size() == 1);
-            if (mergeable && ba.back() == s_a * n && bb.back() == s_b * n && bc.back() == s_c * n) {
+            const long long s_s = pb >= 0 ? wss[pb] : 0;
+            if (mergeable && ba.back() == s_a * n && bb.back() == s_b * n && bc.back() == s_c * n && batch_scales.back() == s_s * n) {
                 bd.back() *= n;
+                batch_scales.back() = s_s;
                 ba.back() = s_a;
                 bb.back() = s_b;
                 bc.back() = s_c;
             } else {
                 bd.push_back(n);
+                batch_scales.push_back(s_s);
                 ba.push_back(s_a);
                 bb.push_back(s_b);
                 bc.push_back(s_c);
@@ -1028,6 +1122,8 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         p->seq = true;
         g.splits = 1;
         g.k_per_split = g.K;
+    } else if (integer_weights(k, *p, own, scale_axis, batch_scales)) {
+        plan_staged(g);
     } else {
         plan_tiles(g, wide);
     }

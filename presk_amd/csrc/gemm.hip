@@ -492,27 +492,6 @@ __device__ __forceinline__ f32x4 mfma<kF32>(float a, float b, f32x4 acc) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
 }
 
-// The stored value of an output element (as store_out computes it).
-template <int ST>
-__device__ __forceinline__ typename St<ST>::S round_out(float sum, bool has_bias, float bias, bool& ovf) {
-    if constexpr (ST == kF32) {
-        return has_bias ? sum + bias : sum;
-    } else if constexpr (ST == kBF16) {
-        unsigned short h = pk_f32_to_bf16(sum);
-        if (has_bias) h = pk_f32_to_bf16(pk_bf16_to_f32(h) + bias);
-        return h;
-    } else {
-        ovf |= pk_overflows_f16(sum);
-        unsigned short h = pk_f32_to_f16(sum);
-        if (has_bias) {
-            const float v = pk_f16_to_f32(h) + bias;
-            ovf |= pk_overflows_f16(v);
-            h = pk_f32_to_f16(v);
-        }
-        return h;
-    }
-}
-
 // Wait until the k-block a stage is about to be read from has landed, with
 // `later` blocks issued after it (NL loads a thread each) still in flight.
 template <int NL, int L>
@@ -1303,9 +1282,9 @@ hipError_t launch_typed(const GemmArgs& g, hipStream_t stream) {
     // contiguous, else the rows) to hold whole aligned vectors
     const bool fast = g.a_vec && g.b_vec;
     hipError_t e;
-    if (stream_fits(g)) return stream_launch<ST>(g, stream);
-    if (ST == kF32 && g.split3) {
-        e = gemm_split_launch(g, stream);
+    if (!g.b_bits && !g.staged && stream_fits(g)) return stream_launch<ST>(g, stream);
+    if (g.b_bits || g.staged || (ST == kF32 && g.split3)) {
+        e = g.b_bits ? gemm_quant_launch(g, stream) : g.staged ? gemm_ragged_launch(g, stream) : gemm_split_launch(g, stream);
         if (e != hipSuccess || g.splits <= 1) return e;
         split_reduce_kernel<ST><<<(unsigned)((g.M * g.N + 255) / 256), 256, 0, stream>>>(g);
         return hipGetLastError();

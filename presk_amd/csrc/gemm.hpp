@@ -31,6 +31,11 @@ struct GemmArgs {
     int bm;                         // tile rows: 128, or 256 (eight-wave tiles)
     int bn;                         // tile columns: 256, 128, 96 or 64
     bool eight;                     // 128-row tiles of eight waves: 128 x 128, or 128 x 96 in f32 (256-row tiles always have eight)
+    const float* scales;            // an integer B's scales (gemm_quant.hip): column n of batch entry (i_d) at n*ss_n + sum i_d*ss_b[d]
+    long long ss_n, ss_b[3];
+    int b_bits;                     // 8 or 4: B is integer weights, from element b_elem; else 0
+    long long b_elem;
+    bool staged;                    // 16-bit operands staged through registers (gemm_ragged.hip), bm x bn tiles
     bool split3;                    // f32 on the bf16 matrix cores (gemm_split.hip): 128 rows, 192, 128 (eight or four waves) or 64 columns
     bool stream;                    // K of at most two k-blocks may stream B's tiles across a kept A panel
 };
@@ -41,6 +46,14 @@ hipError_t gemm_launch(const GemmArgs& g, hipStream_t stream);
 // the split-K partials' reduction is the caller's
 bool gemm_split_fits(const GemmArgs& g);
 hipError_t gemm_split_launch(const GemmArgs& g, hipStream_t stream);
+
+// 16-bit products staged through registers: operands whose vectors end inside
+// a row, or few rows (gemm_ragged.hip)
+bool gemm_ragged_fits(const GemmArgs& g);
+hipError_t gemm_ragged_launch(const GemmArgs& g, hipStream_t stream);
+// integer weights as B (b_bits), A in 16-bit or f32 storage (gemm_quant.hip)
+bool gemm_quant_fits(const GemmArgs& g);
+hipError_t gemm_quant_launch(const GemmArgs& g, hipStream_t stream);
 
 // EXACT mode: each output its products' running sum in index order, the
 // product and the sum rounded to f32 (gemm_seq.hip); no split
