@@ -876,4 +876,211 @@ bool generate_hip(const Kernel& k, Generated* out, std::string* err, bool fast_f
     return true;
 }
 
+namespace {
+
+// The perfect nest at the top of a kernel of one statement.
+bool perfect_nest(const Kernel& k, std::vector<const Stmt*>* loops, const std::vector<const Stmt*>** body) {
+    const std::vector<const Stmt*>* level = &k.body;
+    while (level->size() == 1 && (*level)[0]->kind == Stmt::For) {
+        loops->push_back((*level)[0]);
+        level = &(*level)[0]->body;
+    }
+    *body = level;
+    return !loops->empty();
+}
+
+int flat_width(Ty t) { return t == Ty::F32 ? 4 : t == Ty::BF16 || t == Ty::F16 ? 8 : 0; }
+
+}  // namespace
+
+bool flat_nest(const Kernel& k, FlatNest* out) {
+    std::vector<const Stmt*> loops;
+    const std::vector<const Stmt*>* body = nullptr;
+    if (!k.arith.empty() || k.n_quant() || k.output.ty != k.dtype || !flat_width(k.output.ty) || !perfect_nest(k, &loops, &body))
+        return false;
+    const auto& dims = k.output.dims;
+    if (loops.size() != dims.size()) return false;
+    std::map<int, int64_t> bounds;
+    int64_t n = 1;
+    for (size_t d = 0; d < dims.size(); ++d) {
+        if (loops[d]->bound != dims[d]) return false;
+        bounds[loops[d]->var] = dims[d];
+        n *= dims[d];
+    }
+    auto own = [&](const std::vector<const Expr*>& ix, const std::vector<int64_t>& shape) {
+        if (ix.size() != loops.size() || shape != dims) return false;
+        for (size_t d = 0; d < ix.size(); ++d)
+            if (ix[d]->kind != Expr::Iv || ix[d]->id != loops[d]->var) return false;
+        return true;
+    };
+    std::vector<bool> same(k.inputs.size(), true);
+    std::vector<const Expr*> lds;
+    int stores = 0;
+    for (auto s : *body) {
+        if (s->kind == Stmt::Set) {
+            loads_of(s->value, lds);
+        } else if (s->kind == Stmt::Store && s->buf == k.out_buf() && own(s->index, dims)) {
+            ++stores;
+            loads_of(s->value, lds);
+        } else {
+            return false;
+        }
+    }
+    if (stores != 1 || (*body).back()->kind != Stmt::Store) return false;
+    for (auto e : lds) {
+        if (e->id == k.out_buf()) return false;
+        if (!own(e->kids, k.buf(e->id).dims)) same[e->id] = false;
+        // every element the nest names is in bounds (its loads may be moved)
+        if (!in_bounds(k, e->id, e->kids, bounds)) return false;
+    }
+    // a scalar carried from one iteration to the next
+    std::set<std::string> def, exp;
+    for (auto l : loops) def.insert("i" + std::to_string(l->var));
+    exposed(*body, def, exp);
+    if (!exp.empty()) return false;
+    const int want = flat_width(k.output.ty);
+    if ((double)n < 65536.0 * want || loops.back()->bound % want) return false;
+    out->vec = want;
+    out->numel = n;
+    out->same = same;
+    return true;
+}
+
+bool generate_chain(const std::vector<const Kernel*>& kernels, const std::vector<std::vector<int>>& from, Generated* out,
+                    std::vector<std::pair<int, int>>* slots, std::string* err) {
+    FlatNest f0;
+    if (kernels.empty() || !flat_nest(*kernels[0], &f0)) {
+        *err = "E10001: not a flat nest";
+        return false;
+    }
+    const std::string V = std::to_string(f0.vec), total = std::to_string(f0.numel / f0.vec) + "LL";
+    std::string decl, loads, work, params, args;
+    bool guarded = false, used_fast = false;
+    slots->clear();
+    for (size_t j = 0; j < kernels.size(); ++j) {
+        const Kernel& k = *kernels[j];
+        FlatNest f;
+        if (!flat_nest(k, &f) || f.vec != f0.vec || f.numel != f0.numel || k.output.ty != kernels[0]->output.ty) {
+            *err = "E10001: nests of different shapes";
+            return false;
+        }
+        Printer P(k);
+        P.fast_fns = true;
+        std::vector<const Stmt*> loops;
+        const std::vector<const Stmt*>* body = nullptr;
+        perfect_nest(k, &loops, &body);
+        const std::string J = std::to_string(j), OT = elem_type(k.output.ty);
+        guarded = guarded || k.guarded();
+        // the pointers this kernel still reads or writes
+        std::string ptrs;
+        for (int b = 0; b <= (int)k.inputs.size(); ++b) {
+            if (b < (int)k.inputs.size() && from[j][b] >= 0) continue;
+            const std::string q = "q" + std::to_string(slots->size());
+            params += ", " + P.ptr_type(b) + " __restrict__ " + q;
+            args += ", (" + P.ptr_type(b) + ")a.buf[" + std::to_string(slots->size()) + "]";
+            ptrs += "        " + P.ptr_type(b) + " pb" + std::to_string(b) + " = " + q + "; (void)pb" + std::to_string(b) + ";\n";
+            slots->push_back({(int)j, b});
+        }
+        if ((int)slots->size() > kMaxBufs) {
+            *err = "E10001: more than " + std::to_string(kMaxBufs) + " buffers";
+            return false;
+        }
+        // the thread's first element as the kernel's own indices
+        std::string index = "        long long t = t0;\n";
+        for (size_t d = loops.size(); d-- > 0;) {
+            const bool last = d + 1 == loops.size();
+            const std::string v = "i" + std::to_string(loops[d]->var);
+            const std::string n = std::to_string(last ? loops[d]->bound / f.vec : loops[d]->bound) + "LL";
+            index += "        long long " + v + " = " + (d ? "t % " + n : std::string("t")) + (last ? " * " + V + "LL" : "") + "; (void)" + v + ";";
+            index += d ? " t /= " + n + ";\n" : "\n";
+        }
+        // the vectors it reads, all loaded before any kernel's work; an
+        // earlier kernel's output is that kernel's registers
+        const int iv = loops.back()->var;
+        std::vector<const Expr*> lds;
+        for (auto s : *body) {
+            for (auto e : s->index) loads_of(e, lds);
+            if (s->value) loads_of(s->value, lds);
+        }
+        std::string pre, names;
+        for (auto e : lds) {
+            const int b = e->id;
+            const Ty ty = k.buf(b).ty;
+            if (ty == Ty::E8M15 || ty_quant(ty)) continue;
+            bool unit = !e->kids.empty();
+            for (size_t p = 0; p < e->kids.size(); ++p) {
+                Affine a = affine_of(e->kids[p]);
+                const int64_t c = a.coef.count(iv) ? a.coef[iv] : 0;
+                if (!a.ok || c != (p + 1 == e->kids.size() ? 1 : 0)) unit = false;
+            }
+            const std::string key = std::to_string(b) + "|" + index_key(e->kids);
+            if (!unit || P.pre.count(key)) continue;
+            const int n = (int)P.pre.size();
+            const std::string T = elem_type(ty), local = "pre" + std::to_string(n);
+            if (b < (int)k.inputs.size() && from[j][b] >= 0) {
+                names += "        " + T + " (&" + local + ")[" + V + "] = post_" + std::to_string(from[j][b]) + ";\n";
+            } else {
+                const std::string g = "pre_" + J + "_" + std::to_string(n);
+                const int bytes = f.vec * elem_bytes(ty);
+                decl += "    " + T + " " + g + "[" + V + "];\n";
+                names += "        " + T + " (&" + local + ")[" + V + "] = " + g + ";\n";
+                pre += "        { const " + T + "* p_ = " + P.ptr(b) + " + " + P.offset(b, e->kids) + ";\n";
+                if (bytes % 16 == 0) {
+                    pre += "          if ((((unsigned long long)p_) & 15ULL) == 0) {\n";
+                    pre += "#pragma unroll\n            for (int c = 0; c < " + std::to_string(bytes / 16) +
+                           "; ++c) { pk_u32x4 w_ = ((const pk_u32x4*)p_)[c]; __builtin_memcpy((char*)" + g + " + 16 * c, &w_, 16); }\n";
+                    pre += "          } else {\n#pragma unroll\n            for (int u = 0; u < " + V + "; ++u) " + g + "[u] = p_[u];\n          }\n";
+                } else {
+                    pre += "#pragma unroll\n          for (int u = 0; u < " + V + "; ++u) " + g + "[u] = p_[u];\n";
+                }
+                pre += "        }\n";
+            }
+            P.pre[key] = n;
+        }
+        if (!pre.empty()) loads += "    {\n" + index + ptrs + pre + "    }\n";
+        const Stmt* ost = body->back();
+        P.post_key = index_key(ost->index);
+        decl += "    " + OT + " post_" + J + "[" + V + "];\n";
+        work += "    {\n" + index + ptrs + names;
+        for (int v = 0; v < k.nreal; ++v) work += "        " + P.A + " s" + std::to_string(v) + " = 0; (void)s" + std::to_string(v) + ";\n";
+        const std::string v = "i" + std::to_string(iv);
+        work += "        " + OT + " (&post)[" + V + "] = post_" + J + ";\n";
+        work += "        const long long " + v + "_0 = " + v + ", o_ = " + P.offset(k.out_buf(), ost->index) + ";\n";
+        work += "#pragma unroll\n        for (int u = 0; u < " + V + "; ++u) {\n            " + v + " = " + v + "_0 + u;\n";
+        P.stmts(*body, 3, work);
+        work += "        }\n";
+        const int chunks = elem_bytes(k.output.ty) * f.vec / 16;
+        // the stored words hidden from the optimiser: a later kernel's use of
+        // them is not simplified together with what made them
+        work += "#pragma unroll\n        for (int c = 0; c < " + std::to_string(chunks) + "; ++c) { pk_u32x4 w_; __builtin_memcpy(&w_, (const char*)post + 16 * c, 16); "
+                "asm volatile(\"\" : \"+v\"(w_)); __builtin_memcpy((char*)post + 16 * c, &w_, 16); }\n";
+        work += "        { " + OT + "* p_ = " + P.ptr(k.out_buf()) + " + o_;\n";
+        work += "          if ((((unsigned long long)p_) & 15ULL) == 0) {\n";
+        work += "#pragma unroll\n            for (int c = 0; c < " + std::to_string(chunks) +
+                "; ++c) { pk_u32x4 w_; __builtin_memcpy(&w_, (const char*)post + 16 * c, 16); ((pk_u32x4*)p_)[c] = w_; }\n";
+        work += "          } else {\n#pragma unroll\n            for (int u = 0; u < " + V + "; ++u) p_[u] = post[u];\n          }\n        }\n    }\n";
+        used_fast = used_fast || P.used_fast;
+        if (!P.err.empty()) {
+            *err = "E10001: " + P.err;
+            return false;
+        }
+    }
+    Phase ph;
+    ph.fn = "pk_chain_" + std::to_string(kernels.size());
+    ph.bounds.push_back(f0.numel / f0.vec);
+    std::string src = "#include \"devfmt.hpp\"\n";
+    src += "struct PkArgs { void* buf[" + std::to_string(kMaxBufs) + "]; unsigned* flag; long long lo, hi; };\n";
+    src += "typedef unsigned int pk_u32x4 __attribute__((ext_vector_type(4)));\n";
+    src += "__device__ __forceinline__ void " + ph.fn + "_body(const PkArgs& a" + params + ") {\n";
+    src += "    const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;\n";
+    src += "    if (t0 >= " + total + ") return;\n    bool ovf = false; (void)ovf;\n" + decl + loads + work;
+    if (guarded) src += "    if (ovf) atomicOr(a.flag, 1u);\n";
+    src += "}\n";
+    src += "extern \"C\" __global__ void __launch_bounds__(256) " + ph.fn + "(PkArgs a) { " + ph.fn + "_body(a" + args + "); }\n";
+    out->src = src;
+    out->phases = {ph};
+    out->fast_fns = used_fast;
+    return true;
+}
+
 }  // namespace presk

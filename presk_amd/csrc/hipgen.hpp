@@ -43,6 +43,27 @@ struct Generated {
 // its bits.
 bool generate_hip(const Kernel& k, Generated* out, std::string* err, bool fast_fns = false);
 
+// A nest that is one elementwise pass: its loops are the output's axes in
+// order, all on the grid, `vec` consecutive elements a thread, and its one
+// store is unconditional, so thread t writes elements [t vec, t vec + vec) of
+// the flat output.  `same`: the inputs it reads at the output's own index only.
+struct FlatNest {
+    int vec = 0;
+    int64_t numel = 0;
+    std::vector<bool> same;
+};
+bool flat_nest(const Kernel& k, FlatNest* out);
+
+// One launch for a run of such nests over one element count and vector width:
+// kernels[j] after kernels[j - 1] in each thread.  from[j][b]: the earlier
+// kernel whose output input b is (its `same`), taken from that kernel's
+// registers, as stored; -1: memory.  Every kernel's output is written.  The
+// pointers are the kernels' buffers in order, inputs then output, without the
+// inputs taken from registers (`slots`: kernel and buffer of each).  FAST mode's
+// exp and erf.
+bool generate_chain(const std::vector<const Kernel*>& kernels, const std::vector<std::vector<int>>& from, Generated* out,
+                    std::vector<std::pair<int, int>>* slots, std::string* err);
+
 // The argument block every printed phase takes (by value).
 struct PhaseArgs {
     void* buf[kMaxBufs];

@@ -226,7 +226,20 @@ struct presk_hip_kernel {
     // a class kernel's scratch for presk_hip_run, allocated on first use
     mutable void* work = nullptr;
     int mode = PRESK_HIP_EXACT;
+    // printed chains that begin with this kernel (a recorded batch's graph),
+    // loaded as its own module is and unloaded with it: a graph in flight may
+    // still be running their code when its batch is released
+    struct Chain {
+        std::string src;
+        hipModule_t module;
+        hipFunction_t fn;
+    };
+    mutable std::vector<Chain> chains;
 };
+
+// The most chains a kernel keeps; a further one is launched kernel by kernel.
+constexpr size_t kMaxChains = 16;
+std::mutex g_chains_mu;
 
 extern "C" {
 
@@ -425,6 +438,7 @@ int64_t presk_hip_kernel_text(const presk_hip_kernel* h, char* buf, size_t cap) 
 void presk_hip_release(presk_hip_kernel* h) {
     if (!h) return;
     if (h->module) hipModuleUnload(h->module);
+    for (const auto& c : h->chains) hipModuleUnload(c.module);
     if (h->work) hipFree(h->work);
     delete h;
 }
@@ -510,12 +524,35 @@ struct presk_hip_batch {
     std::vector<Item> items;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    // the graph's launches: an item, or (`fn` set) a run of `count`
+    // elementwise items from `first` in one printed kernel
+    struct Unit {
+        int first = 0, count = 1;
+        hipFunction_t fn = nullptr;
+        unsigned grid = 0;
+        PhaseArgs args{};
+    };
+    std::vector<Unit> units;
 
     void drop_graph() {
         if (exec) hipGraphExecDestroy(exec);
         if (graph) hipGraphDestroy(graph);
         exec = nullptr;
         graph = nullptr;
+        units.clear();
+    }
+    int run_units(hipStream_t s) const {
+        for (const Unit& u : units) {
+            if (!u.fn) {
+                if (int rc = run_one(items[u.first], s)) return rc;
+                continue;
+            }
+            PhaseArgs a = u.args;
+            void* params[] = {&a};
+            hipError_t e = hipModuleLaunchKernel(u.fn, u.grid, 1, 1, 256, 1, 1, 0, s, params, nullptr);
+            if (e != hipSuccess) return hip_fail(e, "hipModuleLaunchKernel");
+        }
+        return PRESK_HIP_OK;
     }
     static int run_one(const Item& it, hipStream_t s) {
         if (!it.k && it.rate >= 0.0) {
@@ -540,6 +577,124 @@ namespace {
 
 constexpr int kMaxBranches = 8;
 constexpr bool kBranchesOn = false;
+
+// Whether byte ranges [a, a + na) and [b, b + nb) meet.
+bool meet(const void* a, int64_t na, const void* b, int64_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + (uintptr_t)nb && y < x + (uintptr_t)na;
+}
+
+int64_t buffer_bytes(const BufSpec& s) { return s.numel() * ty_bytes(s.ty); }
+
+// A printed chain's function, from those its first kernel holds; null when it
+// cannot be had (its kernels are then launched one by one).
+hipFunction_t chain_function(const presk_hip_kernel* h, const Generated& g) {
+    std::lock_guard<std::mutex> lock(g_chains_mu);
+    for (const auto& c : h->chains)
+        if (c.src == g.src) return c.fn;
+    std::vector<char> code;
+    std::string err;
+    presk_hip_kernel::Chain c{g.src, nullptr, nullptr};
+    if (h->chains.size() >= kMaxChains || (g.phases[0].bounds[0] + 255) / 256 > 0x7fffffffLL ||
+        !build_code_object(g.src, &code, &err) || hipModuleLoadData(&c.module, code.data()) != hipSuccess)
+        return nullptr;
+    if (hipModuleGetFunction(&c.fn, c.module, g.phases[0].fn.c_str()) != hipSuccess) {
+        (void)hipModuleUnload(c.module);
+        return nullptr;
+    }
+    h->chains.push_back(c);
+    return c.fn;
+}
+
+// The batch's launches as the graph takes them: runs of elementwise nests
+// over the same elements, each reading one of the run's earlier outputs,
+// become one launch that writes every output and takes what it reads of them
+// from registers.  Such a run is bound by its bytes and by the ~2 us a launch
+// takes to fill and drain the chip: LayerNorm's reverse mode in bf16 at
+// 16384 x 384, 20 launches over 12.6 MB matrices 126 -> 101 us; the
+// attention gradient's broadcast, sub and mul, div over 100 MB matrices
+// saves two of its eight passes, 499 -> 458 us for the whole call.
+// A thread reads only what it wrote itself: the later nest reads the earlier
+// one's whole output at its own index, and the bytes it writes meet nothing
+// that the run reads or writes.  FAST only: the compiler may order a product's
+// operands differently in the longer kernel, and the sign of a NaN is that of
+// the first one.
+void plan_units(presk_hip_batch& b, bool chains) {
+    constexpr size_t kMaxChain = 6;
+    b.units.clear();
+    const size_t n = b.items.size();
+    auto flat = [&](const presk_hip_batch::Item& it, FlatNest* f) {
+        if (!it.k || it.k->mode != PRESK_HIP_FAST || it.k->plan || it.k->gen.phases.size() != 1) return false;
+        const int64_t split = parallel_outer(*it.k->k);
+        if (it.lo != 0 || it.hi != (split > 0 ? split : 0)) return false;
+        return flat_nest(*it.k->k, f);
+    };
+    for (size_t i = 0; i < n;) {
+        presk_hip_batch::Unit u;
+        u.first = (int)i;
+        FlatNest f0;
+        std::vector<std::vector<int>> from;
+        size_t count = 1, slots = 0;
+        if (chains && flat(b.items[i], &f0)) {
+            const Kernel& k0 = *b.items[i].k->k;
+            from.push_back(std::vector<int>(k0.inputs.size(), -1));
+            slots = k0.inputs.size() + 1;
+            for (; count < kMaxChain && i + count < n; ++count) {
+                const auto& it = b.items[i + count];
+                FlatNest f;
+                if (!flat(it, &f) || f.vec != f0.vec || f.numel != f0.numel) break;
+                const Kernel& k = *it.k->k;
+                if (k.output.ty != k0.output.ty) break;
+                const void* out = it.bufs[k.out_buf()];
+                const int64_t out_bytes = buffer_bytes(k.output);
+                std::vector<int> link(k.inputs.size(), -1);
+                bool ok = true, linked = false;
+                size_t need = 1;
+                for (size_t q = 0; q < k.inputs.size() && ok; ++q) {
+                    if (meet(it.bufs[q], buffer_bytes(k.inputs[q]), out, out_bytes)) ok = false;
+                    for (size_t e = 0; e < count && ok; ++e) {
+                        const auto& pe = b.items[i + e];
+                        const Kernel& ke = *pe.k->k;
+                        const void* po = pe.bufs[ke.out_buf()];
+                        if (!meet(it.bufs[q], buffer_bytes(k.inputs[q]), po, buffer_bytes(ke.output))) continue;
+                        if (po != it.bufs[q] || !f.same[q] || k.inputs[q].ty != ke.output.ty) ok = false;
+                        link[q] = (int)e;
+                        linked = true;
+                    }
+                    if (link[q] < 0) ++need;
+                }
+                // nothing of the run reads or writes the bytes this one writes
+                for (size_t e = 0; e < count && ok; ++e) {
+                    const auto& pe = b.items[i + e];
+                    const Kernel& ke = *pe.k->k;
+                    for (size_t q = 0; q <= ke.inputs.size(); ++q)
+                        if (meet(pe.bufs[q], buffer_bytes(ke.buf((int)q)), out, out_bytes)) ok = false;
+                    if (k.guarded() && it.bufs[k.flag_slot()] != pe.bufs[ke.flag_slot()]) ok = false;
+                }
+                if (!ok || !linked || slots + need > (size_t)kMaxBufs) break;
+                slots += need;
+                from.push_back(link);
+            }
+        }
+        if (count > 1) {
+            std::vector<const Kernel*> ks;
+            for (size_t e = 0; e < count; ++e) ks.push_back(b.items[i + e].k->k.get());
+            Generated g;
+            std::vector<std::pair<int, int>> where;
+            std::string err;
+            if (generate_chain(ks, from, &g, &where, &err) &&
+                (u.fn = chain_function(b.items[i].k, g))) {
+                u.count = (int)count;
+                u.grid = (unsigned)((g.phases[0].bounds[0] + 255) / 256);
+                for (size_t q = 0; q < where.size(); ++q) u.args.buf[q] = b.items[i + where[q].first].bufs[where[q].second];
+                const Kernel& k0 = *ks[0];
+                u.args.flag = k0.guarded() ? (unsigned*)b.items[i].bufs[k0.flag_slot()] : nullptr;
+            }
+        }
+        i += (size_t)u.count;
+        b.units.push_back(u);
+    }
+}
 
 // The batch's items as the branch planner (branches.hpp) reads them.
 std::vector<BranchStep> branch_steps(const presk_hip_batch& b) {
@@ -640,6 +795,7 @@ int presk_hip_batch_graph_branches(presk_hip_batch* b, int branches) {
         if (it.k)
             if (int rc = prepare_kernel(it.k)) return rc;
     const int n = (int)b->items.size();
+    plan_units(*b, branches == 1);
     std::vector<int> lane;       // each step's capture stream
     std::vector<std::vector<std::pair<int, int>>> waits;   // (stream, step) events each step waits for
     plan_branches(branch_steps(*b), branches, &lane, &waits);
@@ -671,7 +827,7 @@ int presk_hip_batch_graph_branches(presk_hip_batch* b, int branches) {
     }
     int rc = PRESK_HIP_OK;
     if (used == 1) {
-        rc = b->run_each(cs[0]);
+        rc = b->run_units(cs[0]);
     } else {
         // the other streams join the capture from the first one, then each
         // step waits for the last step of every other stream it depends on,
