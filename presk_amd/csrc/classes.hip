@@ -618,9 +618,9 @@ void plan_staged(GemmArgs& g) {
         long long s = 512 / t;
         // few rows: eight 64-deep blocks a split, four where that leaves CUs
         // idle (8 x 4096 x 4096 split 8 12.0 us, 16 12.6); 128-row tiles: a
-        // K of 256, or of 1024 from 96 tiles on (1999 x 1021 x 777, 208 of
-        // them: unsplit 21.1 us, 4 ways 28; 4096 x 65 x 1021, 64: unsplit
-        // 24.2, 4 ways 21.2; int8 weights from 16, their conversion being
+        // K of 256, or of 1024 from 96 tiles on (1999 x 1021 x 777, 112 of
+        // them: unsplit 13.9 us, 4 ways 28.9; 4096 x 65 x 1021, 64: unsplit
+        // 16.3, 4 ways 12.1; int8 weights from 16, their conversion being
         // the longer part of a block: 128 x 4096 x 4096, 32 tiles, 4 ways 22.8
         // us, 16 ways 28.4)
         const long long least = g.bm == 32 ? (t * (nkb / 8) >= 256 ? 8 : 4) : (t < (g.b_bits ? 16 : 96) ? 256 : 1024) / unit;

@@ -8,7 +8,12 @@
 // before they are converted and stored, each loaded again as soon as it has
 // been stored, so a load has a block's time to land.  Vectors are read at any
 // alignment (gfx950's global loads take any byte address); where EDGE, one
-// that crosses the operand's end is read element by element.
+// that runs past its row's end reads what follows there, which no result uses
+// (k past the end is zeroed on the way to LDS), and only one that runs past
+// the operand's last element is read element by element (read so at every
+// row's end, those loads' waits left nothing in flight: 1999 x 1021 x 777 in
+// f16 22.3 us, now 16.5; the f32 gradient [384 x 65] over K 16384 27.2, now
+// 23.7).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -82,6 +87,7 @@ struct StageLoader {
     unsigned rstr, kstr;         // elements between rows and between k
     int last;                    // the tile's last existing row
     long long step;              // elements a k-block
+    long long end;               // one past the operand's last element (EDGE)
     Raw r[NV];
 
     __device__ static __forceinline__ int swz(int k) {
@@ -99,20 +105,22 @@ struct StageLoader {
         return KC ? slot / VPR : (slot % VPR) * V;
     }
     // element `off` from the operand's first, rows from row0 (row0 < rows),
-    // strides in elements.  Rows past the operand read its last row (or last
-    // whole vector): the results of such rows are never stored.
-    __device__ __forceinline__ void init(const void* p, long long off, int rows, long long rs, long long ks, int row0, int k0) {
+    // strides in elements, K of the whole operand.  Rows past it read its last
+    // row (or last whole vector): the results of such rows are never stored.
+    __device__ __forceinline__ void init(const void* p, long long off, int rows, long long rs, long long ks, int row0, int k0,
+                                         long long K) {
         base = (const char*)p;
         origin = off + (long long)row0 * rs + (long long)k0 * ks;
         step = (long long)BK * ks;
         rstr = (unsigned)rs;
         kstr = (unsigned)ks;
         last = rows - 1 - row0;
+        end = off + (long long)(rows - 1) * rs + (K - 1) * ks + 1;
 #pragma unroll
         for (int q = 0; q < NV; ++q) {
             const int row = row_of(q);
             if (KC) voff[q] = (unsigned)(row < last ? row : last) * rstr + (unsigned)k_of(q);
-            else voff[q] = (unsigned)k_of(q) * kstr + (unsigned)(EDGE || row + V - 1 <= last ? row : last - (V - 1));
+            else voff[q] = (unsigned)k_of(q) * kstr + (unsigned)(EDGE ? (row < last ? row : last) : row + V - 1 <= last ? row : last - (V - 1));
         }
     }
     __device__ __forceinline__ Raw vec(unsigned off) const {
@@ -130,26 +138,27 @@ struct StageLoader {
     }
     // vector q of the block at the origin, `left` of whose k exist (at least
     // one); k past them reads the row's first k instead and is zeroed by
-    // store1, so that the loads need no branch (EDGE: where the vector is
-    // not whole, its elements one by one, those past the end zero)
+    // store1, so that the loads need no branch (EDGE: but for a vector past
+    // the operand's last element, or of int4 from the middle of a byte; SURE:
+    // a whole block, and no vector of it is past the operand)
+    template <bool SURE = false>
     __device__ __forceinline__ void load1(int q, int left) {
         const int k = k_of(q);
+        const unsigned back = KC ? (unsigned)k : (unsigned)k * kstr;
+        const unsigned off = left >= BK || k < left ? voff[q] : voff[q] - back;
         if constexpr (EDGE) {
-            const int row = row_of(q);
-            bool whole = KC ? left >= BK || k + V <= left : row + V - 1 <= last && (left >= BK || k < left);
-            if (OP == kOpQ4) whole = whole && (((unsigned)(origin & 1) + voff[q]) & 1) == 0;
-            if (whole) {
-                r[q] = vec(voff[q]);
+            const long long at = origin + off;
+            if ((SURE || (KC && left >= BK) || at + V <= end) && (OP != kOpQ4 || (((unsigned)(origin & 1) + off) & 1) == 0)) {
+                r[q] = vec(off);
             } else {
                 Raw x = {};
 #pragma unroll
                 for (int e = 0; e < V; ++e)
-                    if (KC ? k + e < left : row + e <= last && k < left) put(x, e, origin + voff[q] + e);
+                    if (at + e < end) put(x, e, at + e);
                 r[q] = x;
             }
         } else {
-            const unsigned back = KC ? (unsigned)k : (unsigned)k * kstr;
-            r[q] = vec(left >= BK || k < left ? voff[q] : voff[q] - back);
+            r[q] = vec(off);
         }
     }
     __device__ __forceinline__ void load(int left) {
@@ -168,10 +177,16 @@ struct StageLoader {
             const int k = slot / VPR, c = (slot % VPR) * V / 8;
             off = k * ROWS * 2 + ((c ^ swz(k)) << 4);
         }
-        const bool none = !EDGE && left < BK && k_of(q) >= left;    // a whole vector of k past the end
+        const bool none = left < BK && k_of(q) >= left;    // a whole vector of k past the end
+        // the elements of the vector whose k exists
+        const int some = EDGE && KC && left < BK ? left - k_of(q) : V;
         if constexpr (OP == kOpF32) {
             f32x4 x = __builtin_bit_cast(f32x4, r[q]);
             if (none) x = f32x4{};
+            if (EDGE && KC && left < BK) {
+#pragma unroll
+                for (int e = 1; e < V; ++e) x[e] = e < some ? x[e] : 0.f;
+            }
             off += (slot & 1) * 8;
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
@@ -185,9 +200,25 @@ struct StageLoader {
                 }
             }
         } else if constexpr (OP == kOpHalf) {
-            *(u32x4*)(tile + off) = none ? u32x4{} : r[q];
+            u32x4 w = none ? u32x4{} : r[q];
+            if (EDGE && KC && left < BK) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] &= some >= 2 * i + 2 ? ~0u : some == 2 * i + 1 ? 0xffffu : 0u;
+            }
+            *(u32x4*)(tile + off) = w;
         } else {
-            const Raw w = none ? Raw{} : r[q];
+            Raw w = none ? Raw{} : r[q];
+            if constexpr (EDGE && KC) {
+                if (left < BK && some < V) {
+                    const int bits = (some > 0 ? some : 0) * (OP == kOpQ8 ? 8 : 4);
+                    if constexpr (OP == kOpQ8) {
+                        w[0] &= bits >= 32 ? ~0u : (1u << bits) - 1;
+                        w[1] &= bits >= 64 ? ~0u : bits > 32 ? (1u << (bits - 32)) - 1 : 0u;
+                    } else {
+                        w &= (1u << bits) - 1;
+                    }
+                }
+            }
             u32x4 h;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -301,8 +332,8 @@ __global__ void __launch_bounds__(64 * NW, 2) staged_gemm_kernel(GemmArgs g) {
     const int nk = (kend - kbeg + BK - 1) / BK;
     LA la;
     LB lb;
-    la.init(g.A, a_off, M, g.sa_m, g.sa_k, m0, kbeg);
-    lb.init(g.B, b_off + (QUANT ? g.b_elem : 0), N, g.sb_n, g.sb_k, n0, kbeg);
+    la.init(g.A, a_off, M, g.sa_m, g.sa_k, m0, kbeg, g.K);
+    lb.init(g.B, b_off + (QUANT ? g.b_elem : 0), N, g.sb_n, g.sb_k, n0, kbeg, g.K);
     if (nk > 0) {
         la.load(kend - kbeg);
         lb.load(kend - kbeg);
@@ -326,7 +357,7 @@ __global__ void __launch_bounds__(64 * NW, 2) staged_gemm_kernel(GemmArgs g) {
     // into the other stage, one vector after every few MFMAs; LOAD, the loads
     // of the block after it, `lleft` of its k existing
     auto block = [&](int kt, auto store, auto load, int sleft, int lleft) {
-        constexpr bool STORE = decltype(store)::value, LOAD = decltype(load)::value;
+        constexpr bool STORE = decltype(store)::value, LOAD = decltype(load)::value > 0, SURE = decltype(load)::value > 1;
         char* const cur = smem + (kt & 1) * STAGE;
         char* const nx = smem + ((kt & 1) ^ 1) * STAGE;
 #pragma unroll
@@ -357,10 +388,10 @@ __global__ void __launch_bounds__(64 * NW, 2) staged_gemm_kernel(GemmArgs g) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (done < LA::NV) {
                     la.store1(nx, done, sleft);
-                    if (LOAD) la.load1(done, lleft);
+                    if (LOAD) la.template load1<SURE>(done, lleft);
                 } else {
                     lb.store1(nx + LA::BYTES, done - LA::NV, sleft);
-                    if (LOAD) lb.load1(done - LA::NV, lleft);
+                    if (LOAD) lb.template load1<SURE>(done - LA::NV, lleft);
                 }
                 ++done;
             };
@@ -410,12 +441,19 @@ __global__ void __launch_bounds__(64 * NW, 2) staged_gemm_kernel(GemmArgs g) {
             lb.origin += lb.step;
         }
     };
-    const std::integral_constant<bool, true> yes;
-    const std::integral_constant<bool, false> no;
+    const std::integral_constant<int, 0> no;
+    const std::integral_constant<int, 1> yes;
+    const std::integral_constant<int, 2> sure;
     int kt = 0;
-    // (the block loaded last may be partial)
-    for (; kt + 3 < nk; ++kt) block(kt, yes, yes, BK, BK);
-    if (kt + 2 < nk) {
+    // All blocks but the last are whole, and a vector that runs past its row
+    // there ends inside the next k's, unless those lie closer than a vector:
+    // then, and for the last, the loads are checked.
+    const bool close = EDGE && ((!AK && la.kstr < LA::V) || (!BKC && lb.kstr < LB::V));
+    if (!close)
+        for (; kt + 3 < nk; ++kt) block(kt, yes, sure, BK, BK);
+    if constexpr (EDGE) {
+        for (; kt + 2 < nk; ++kt) block(kt, yes, yes, BK, kend - kbeg - (kt + 2) * BK);
+    } else if (kt + 2 < nk) {
         block(kt, yes, yes, BK, kend - kbeg - (kt + 2) * BK);
         ++kt;
     }

@@ -50,7 +50,7 @@ def call(c, ins, nbytes, lo=0, hi=None, out=None):
 # k-block, ragged in rows, columns or k alone, the few-row tiles whole and
 # ragged, split plans, and sizes below a vector
 SIZES = [(129, 65, 77), (127, 193, 129), (1000, 72, 1021), (264, 100, 63), (300, 40, 2050), (5, 136, 520), (32, 1032, 1100),
-         (31, 129, 4100), (3, 7, 5), (65, 257, 64)]
+         (31, 129, 4100), (3, 7, 5), (65, 257, 64), (300, 5, 1100)]
 
 
 @pytest.mark.gpu
@@ -82,6 +82,34 @@ def test_ragged_and_few_rows_equal_the_tiles(kind, dt, scale, m, n, k, monkeypat
     assert outs[0][1] == outs[1][1]
     differ = np.count_nonzero(outs[0][0] != outs[1][0])
     assert differ == 0, f"{differ} of {outs[0][0].size} outputs differ from the 128 x 128 tiles'"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(140, 70, 77), (129, 71, 1021), (66, 131, 97)])
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("kind", ["nn", "nt", "tn", "tt"])
+def test_what_follows_a_ragged_row_reaches_no_other_output(kind, dt, m, n, k):
+    """Vectors past a row's end hold the next row's elements: infinities and
+    NaN there give NaN in their own rows and columns alone."""
+    hip.init(0)
+    print(f"[staged] {kind} {dt} {m}x{n}x{k} with NaN", flush=True)
+    from oracle import kernel_text as kt
+    low = nest(kind, m, n, k, dt)
+    rng = np.random.default_rng(m + n + k)
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    rows, cols = [1, m // 2, m - 1], [2, n - 2]
+    x[rows[0], 0], x[rows[1], : 3], x[rows[2], k - 1] = np.nan, np.inf, -np.inf
+    w[0, cols[0]], w[k - 1, cols[1]] = np.nan, np.inf
+    stored = {"nn": (x, w), "nt": (x, w.T), "tn": (x.T, w), "tt": (x.T, w.T)}[kind]
+    dims = [tuple(b.dims) for b in kt.parse_kernel(low.text).inputs]
+    assert dims == [q.shape for q in stored], dims
+    c = hip.Compiled(low.text, dt, low.lanes, hip.FAST)
+    out, _ = call(c, [hip.DeviceBuffer.of(fmt.encode(np.ascontiguousarray(q), dt)) for q in stored], (4 if dt == "f32" else 2) * m * n)
+    got = fmt.decode(out.download(np.float32 if dt == "f32" else np.uint16), dt).reshape(m, n)
+    with np.errstate(invalid="ignore"):
+        want = fmt.roundtrip(x, dt).astype(np.float64) @ fmt.roundtrip(w, dt).astype(np.float64)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
 
 
 # name -> (nest, the weights' stored axes, the axis their scales run over, the
