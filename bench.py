@@ -24,6 +24,14 @@ sys.path.insert(0, ROOT)
 
 METRIC = "tokens/sec course-GPT fwd+bwd; matmul TFLOP/s as % of MFMA peak"
 PEAK_TFLOPS = {"bf16": 2500.0, "f16": 2500.0, "f32": 157.3}   # MI355X dense MFMA
+
+
+def mfma_peak(dtype: str, order: str) -> float:
+    """The nominal matrix-core rate of a contraction: its storage type's, or,
+    of an f32 one whose operands enter as three bf16 parts (six bf16 products
+    a term), a sixth of bf16's."""
+    return round(PEAK_TFLOPS["bf16"] / 6, 1) if "f32x3" in order else PEAK_TFLOPS.get(dtype, PEAK_TFLOPS["f32"])
+
 HBM_GBS = 8000.0
 DATA = {"gpt-step": "synthetic (seeded ids and targets uniform over the vocabulary, N(0,0.02) weights)",
         "gpt-forward": "synthetic (seeded ids and targets uniform over the vocabulary, N(0,0.02) weights)",
@@ -143,13 +151,14 @@ def measured_peaks() -> dict:
     return out
 
 
-def with_measured(roof: dict, storage: str, peaks) -> dict:
+def with_measured(roof: dict, storage: str, peaks, order: str = "") -> dict:
     """The roofline beside the measured peak of its bound (the vendor figure
     stays `peak` and `frac`)."""
     if not peaks:
         return roof
     if roof["bound"] == "mfma":
-        pm = peaks["mfma_bf16_tflops" if storage in ("bf16", "f16") else "mfma_f32_tflops"]
+        pm = peaks["mfma_bf16_tflops" if storage in ("bf16", "f16") or "f32x3" in order else "mfma_f32_tflops"]
+        pm = round(pm / 6, 1) if "f32x3" in order else pm
     else:
         pm = peaks["hbm_copy_gbs"]
     return dict(roof, peak_measured=pm, frac_of_measured=round(roof["achieved"] / pm, 4))
@@ -296,7 +305,7 @@ def measure(name, dtype, steps, warmup, realize=None, dropout=0.0, adamw=False, 
     traffic = TRAFFIC.get(launch_key(ln))
     if c.flops > 0:
         achieved = c.flops / (ms * 1e-3) / 1e12
-        peak = PEAK_TFLOPS[ln.low.dtype]
+        peak = mfma_peak(ln.low.dtype, ln.compiled.order)
         roof = {"kernel": f"{ln.low.name} [{c.kind}, {c.order}]", "bound": "mfma", "achieved": round(achieved, 2),
                 "peak": peak, "unit": "TFLOP/s", "frac": round(achieved / peak, 4), "traffic": traffic,
                 "ms_per_launch": round(ms, 5), "algorithmic_flops": c.flops}
@@ -307,7 +316,7 @@ def measure(name, dtype, steps, warmup, realize=None, dropout=0.0, adamw=False, 
                 "ms_per_launch": round(ms, 5), "algorithmic_bytes": c.bytes}
     if traffic is None:
         roof["traffic_note"] = "no counter measurement of this kernel on these device sources (profiles/traffic.json)"
-    roof = with_measured(roof, ln.low.dtype, peaks)
+    roof = with_measured(roof, ln.low.dtype, peaks, ln.compiled.order)
     agg = {}
     for l, m in times:
         e = agg.setdefault(l.low.name, {"kernel": l.low.name, "kind": l.compiled.kind, "launches": 0, "ms": 0.0})
@@ -316,8 +325,8 @@ def measure(name, dtype, steps, warmup, realize=None, dropout=0.0, adamw=False, 
     per_kernel = sorted(agg.values(), key=lambda e: -e["ms"])[:16]
     for e in per_kernel:
         e["ms"] = round(e["ms"], 4)
-    # the contractions' time at the MFMA peak of each one's storage type
-    bound_ms = sum(l.compiled.flops / (PEAK_TFLOPS.get(l.low.dtype, PEAK_TFLOPS["f32"]) * 1e12) * 1e3
+    # the contractions' time at the MFMA peak of each one's products
+    bound_ms = sum(l.compiled.flops / (mfma_peak(l.low.dtype, l.compiled.order) * 1e12) * 1e3
                    for l in p.launches if l.compiled.kind == "gemm")
     cfg = dict(cfg, launch="eager" if eager else "hip graph")
     rec = {"value": round(tokens / (ms_step * 1e-3), 1), "unit": "tokens/s", "steps": steps, "warmup": warmup,
@@ -413,7 +422,7 @@ def per_launch_table(p, path, ring_mb: float = 768.0):
         each = ms / n * 1e-3
         gbs = c.bytes / each / 1e9
         tf = c.flops / each / 1e12 if c.flops else 0.0
-        peak = PEAK_TFLOPS.get(ln.low.dtype, PEAK_TFLOPS["f32"])
+        peak = mfma_peak(ln.low.dtype, c.order)
         rows.append(f"| `{head[:160]}` | {c.kind}, {c.order} | {n} | {r} | {each * 1e6:.2f} | {ms * 1e3:.1f} | {c.bytes / 1e6:.1f} | "
                     f"{gbs:.0f} | {100 * gbs / HBM_GBS:.0f} | " + (f"{tf:.1f} | {100 * tf / peak:.0f} |" if c.flops else "| |"))
     rows.append(f"| (all {sum(e[0] for e in agg.values())} launches) | | | | | {total * 1e3:.1f} | | | | | |")
