@@ -15,6 +15,7 @@
 #include <map>
 #include <mutex>
 #include <set>
+#include <utility>
 
 #include "devfmt.hpp"
 #include "executor.hpp"
@@ -109,212 +110,289 @@ bool product_pattern(const Kernel& k, std::vector<int>* vars0, std::vector<int>*
     return vars(load0, vars0) && vars(load1, vars1);
 }
 
-// Whether the nest sums each output's products in index order into one
-// accumulator from zero and stores it (with an epilogue, reads it back and
-// adds the bias, in f32 before the store): every layout point of a contraction does, a nest under
-// a realization's `interleaved` or `chunked` order does not.  The summed
-// loops stand inside the output's, in the order of operand 0's axes, around
-// nothing but `x = %0[..]` and `acc = acc + x * %1[..]`, the accumulators set
-// to zero just outside them.
-bool sequential_sum(const Kernel& k) {
-    std::set<int> out_vars, accs, vaccs;
-    std::function<void(const Expr*, std::set<int>&)> ivs = [&](const Expr* e, std::set<int>& v) {
-        if (e->kind == Expr::Iv) v.insert(e->id);
-        for (auto c : e->kids) ivs(c, v);
-    };
-    std::function<void(const std::vector<const Stmt*>&)> outs = [&](const std::vector<const Stmt*>& body) {
-        for (auto s : body) {
-            for (auto e : s->index) ivs(e, out_vars);
-            outs(s->body);
-        }
-    };
-    outs(k.body);
-    std::vector<int> summed;          // the summed loops, outermost first
-    int stores = 0, terms = 0, biased = 0, read_back = 0;
-    bool ok = true;
-    auto is_load = [&](const Expr* e, int b) {
-        if ((e->kind != Expr::Load && e->kind != Expr::VLoad) || e->id != b) return false;
-        // the summed loops index their axes by themselves
-        for (auto c : e->kids) {
-            std::set<int> v;
-            ivs(c, v);
-            for (int u : v)
-                if (!out_vars.count(u) && c->kind != Expr::Iv) return false;
-        }
-        return true;
-    };
-    auto plain = [](const Expr* e) { return e->kind == Expr::Splat ? e->kids[0] : e; };
-    std::function<void(const std::vector<const Stmt*>&, bool)> walk = [&](const std::vector<const Stmt*>& body, bool inside) {
-        int x = -1;                   // the scalar holding %0's element
-        for (size_t i = 0; ok && i < body.size(); ++i) {
-            const Stmt* s = body[i];
-            if (s->kind == Stmt::For) {
-                const bool sum = !out_vars.count(s->var);
-                if (inside && !sum) ok = false;                 // an output loop inside a summed one
-                if (sum) {
-                    // one chain of summed loops in the nest
-                    if (!inside && !summed.empty()) ok = false;
-                    if (inside && body.size() != 1) ok = false;
-                    summed.push_back(s->var);
-                }
-                walk(s->body, inside || sum);
-            } else if (s->kind == Stmt::Set || s->kind == Stmt::VSet) {
-                const bool vec = s->kind == Stmt::VSet;
-                std::set<int>& as = vec ? vaccs : accs;
-                const Expr* v = plain(s->value);
-                if (!inside && !summed.empty()) {
-                    // the epilogue in f32: the bias added to the sum before
-                    // its store (once an accumulator)
-                    const Expr* e = s->value;
-                    const bool add = (e->kind == Expr::Bin || e->kind == Expr::VBin) && e->op == Op::Add;
-                    if (!add || k.dtype != Ty::F32 || k.inputs.size() != 3 || !as.count(s->var) ||
-                        e->kids[0]->kind != (vec ? Expr::Vv : Expr::Sv) || e->kids[0]->id != s->var) { ok = false; break; }
-                    const Expr* b = plain(e->kids[1]);
-                    if ((b->kind != Expr::Load && b->kind != Expr::VLoad) || b->id != 2) ok = false;
-                    ++biased;
-                    continue;
-                }
-                if (!inside) {
-                    if (v->kind != Expr::Num || v->num != 0 || std::signbit(v->num)) ok = false;
-                    as.insert(s->var);
-                    continue;
-                }
-                if (!vec && is_load(s->value, 0) && !accs.count(s->var)) {
-                    x = s->var;
-                    continue;
-                }
-                const Expr* e = s->value;
-                if ((e->kind != Expr::Bin && e->kind != Expr::VBin) || e->op != Op::Add || !as.count(s->var)) { ok = false; break; }
-                const Expr *a = e->kids[0], *m = e->kids[1];
-                if (a->kind != (vec ? Expr::Vv : Expr::Sv) || a->id != s->var) { ok = false; break; }
-                if ((m->kind != Expr::Bin && m->kind != Expr::VBin) || m->op != Op::Mul || !is_load(m->kids[1], 1)) { ok = false; break; }
-                const Expr* l = plain(m->kids[0]);
-                // the generic `ein` term (1 * x0) * x1: 1 * x0 is x0 exactly
-                if (l->kind == Expr::Bin && l->op == Op::Mul && l->kids[0]->kind == Expr::Num && l->kids[0]->num == 1) l = l->kids[1];
-                if (!(l->kind == Expr::Sv && l->id == x && x >= 0) && !is_load(l, 0)) { ok = false; break; }
-                ++terms;
-            } else if (s->kind == Stmt::Store || s->kind == Stmt::VStore) {
-                if (inside || summed.empty() || s->buf != k.out_buf()) { ok = false; break; }
-                const Expr* v = s->value;
-                if ((v->kind == Expr::Sv && accs.count(v->id)) || (v->kind == Expr::Vv && vaccs.count(v->id))) {
-                    ++stores;
-                    continue;
-                }
-                // the epilogue: the stored element read back, plus the bias
-                const bool add = (v->kind == Expr::Bin || v->kind == Expr::VBin) && v->op == Op::Add;
-                if (!add || k.inputs.size() != 3) { ok = false; break; }
-                const Expr *o = v->kids[0], *b = plain(v->kids[1]);
-                auto same = [&](const std::vector<const Expr*>& p, const std::vector<const Expr*>& q) {
-                    if (p.size() != q.size()) return false;
-                    for (size_t d = 0; d < p.size(); ++d)
-                        if (show_expr(*p[d]) != show_expr(*q[d])) return false;
-                    return true;
-                };
-                if ((o->kind != Expr::Load && o->kind != Expr::VLoad) || o->id != k.out_buf() || !same(o->kids, s->index) ||
-                    (b->kind != Expr::Load && b->kind != Expr::VLoad) || b->id != 2)
-                    ok = false;
-                ++read_back;
-            } else {
-                ok = false;
-            }
-        }
-    };
-    walk(k.body, false);
-    if (biased + read_back != (k.inputs.size() == 3 ? stores : 0)) return false;
-    if (!ok || summed.empty() || stores == 0 || stores != terms || (int)(accs.size() + vaccs.size()) < stores) return false;
-    // the summed loops in the order of operand 0's axes
-    std::vector<int> axes;
-    std::function<bool(const std::vector<const Stmt*>&)> first = [&](const std::vector<const Stmt*>& body) {
-        std::function<bool(const Expr*)> find = [&](const Expr* e) {
-            if ((e->kind == Expr::Load || e->kind == Expr::VLoad) && e->id == 0) {
-                for (auto c : e->kids)
-                    if (c->kind == Expr::Iv && !out_vars.count(c->id)) axes.push_back(c->id);
-                return true;
-            }
-            for (auto c : e->kids)
-                if (find(c)) return true;
-            return false;
-        };
-        for (auto s : body)
-            if ((s->value && find(s->value)) || first(s->body)) return true;
-        return false;
-    };
-    return first(k.body) && axes == summed;
-}
+// What each index of a contraction's operands runs over, as its name and
+// shapes (an `ein`: its product's indices) say: axis d of the output, or
+// -1 - s for the s-th summed axis, numbered as operand 0 carries them.
+struct SumRoles {
+    std::vector<int> x, w, bias;
+    std::vector<int64_t> summed;      // the summed axes' lengths
+};
 
-// The row-wise layout of an f32 contraction (lower.rs:846-905): the output's
-// row set to zero, then for each k every element of it read back, its product
-// added and stored -- in f32 the stored element is the running sum, so these
-// are the same values.
-bool row_wise_sum(const Kernel& k) {
-    if (k.dtype != Ty::F32) return false;
-    std::set<int> out_vars;
-    std::function<void(const std::vector<const Stmt*>&)> outs = [&](const std::vector<const Stmt*>& body) {
-        for (auto s : body) {
-            for (auto e : s->index)
-                if (e->kind == Expr::Iv) out_vars.insert(e->id);
-            outs(s->body);
+// Whether the nest computes just that contraction with each output's products
+// summed in index order into one accumulator from zero, the bias added last
+// -- the tiled kernel's order (gemm_seq.hip).  Every layout point of a
+// contraction does; a nest under a realization's `interleaved` or `chunked`
+// order does not, and neither does a nest that only carries the name.  So
+// nothing is taken from the name: every loop's bound is its axis' length,
+// every operand, bias and store index is its role's, each output element is
+// zeroed, summed, biased and stored once, in that order, and the split loop
+// (`parallel_outer`) runs over the output's first axis.
+//
+// Two forms.  Tiled (lower.rs:906-1139): inside the output's loops, `acc =
+// 0` for each of a tile's accumulators, the summed loops around the products,
+// the stores; the bias is added to an accumulator (f32) or to the stored
+// element read back (narrow types round between).  Row-wise, f32
+// (lower.rs:846-905): the output's row set to zero, then for each k every
+// element of it read back, its product added and stored -- in f32 the stored
+// element is the running sum, so these are the same values.
+class OrderedSum {
+public:
+    OrderedSum(const Kernel& k, const SumRoles& r) : k(k), r(r) {}
+
+    bool holds() {
+        for (int b = 0; b < (int)k.inputs.size(); ++b) {
+            const auto& dims = k.inputs[b].dims;
+            const auto& role = b == 0 ? r.x : b == 1 ? r.w : r.bias;
+            if (dims.size() != role.size()) return false;
+            for (size_t p = 0; p < dims.size(); ++p)
+                if (dims[p] != (role[p] >= 0 ? k.output.dims[role[p]] : r.summed[-1 - role[p]])) return false;
         }
+        const std::vector<const Stmt*>* body = &k.body;
+        while (body->size() == 1 && (*body)[0]->kind == Stmt::For) {
+            if (!enter((*body)[0], &outer)) return false;
+            body = &(*body)[0]->body;
+        }
+        if (body->empty() || outer.empty()) return false;
+        return (*body)[0]->kind == Stmt::For ? row_wise(*body) : tiled(*body);
+    }
+
+private:
+    const Kernel& k;
+    const SumRoles& r;
+    std::vector<int> outer, summed;   // loop variables, outermost first
+    std::map<int, int64_t> bound;     // of the loops around a statement
+
+    // An index c * var + t.
+    struct At {
+        int var = -1;
+        int64_t c = 1, t = 0;
+        bool operator==(const At& o) const { return var == o.var && c == o.c && t == o.t; }
     };
-    outs(k.body);
-    bool ok = true;
-    int zeros = 0, terms = 0, biased = 0;
-    std::vector<int> summed, axes;
-    const int64_t numel = k.output.numel();
-    auto same = [&](const std::vector<const Expr*>& p, const std::vector<const Expr*>& q) {
-        if (p.size() != q.size()) return false;
-        for (size_t d = 0; d < p.size(); ++d)
-            if (p[d]->kind != Expr::Iv || q[d]->kind != Expr::Iv || p[d]->id != q[d]->id) return false;
+    static bool at(const Expr* e, At* a) {
+        *a = At{};
+        if (e->kind == Expr::Bin && e->op == Op::Add && e->kids[1]->kind == Expr::Num && e->kids[1]->integral) {
+            a->t = e->kids[1]->inum;
+            e = e->kids[0];
+            if (e->kind != Expr::Bin) return false;
+        }
+        if (e->kind == Expr::Bin && e->op == Op::Mul && e->kids[1]->kind == Expr::Num && e->kids[1]->integral) {
+            a->c = e->kids[1]->inum;
+            e = e->kids[0];
+        }
+        a->var = e->id;
+        return e->kind == Expr::Iv && a->c >= 1 && a->t >= 0 && a->t < a->c;
+    }
+    static bool at(const std::vector<const Expr*>& ix, std::vector<At>* out) {
+        out->clear();
+        for (auto e : ix) {
+            At a;
+            if (!at(e, &a)) return false;
+            out->push_back(a);
+        }
         return true;
+    }
+    bool enter(const Stmt* loop, std::vector<int>* vars) {
+        vars->push_back(loop->var);
+        return bound.emplace(loop->var, loop->bound).second;
+    }
+    // the summed loops from `loop` in, to the statements they surround
+    const std::vector<const Stmt*>* enter_sum(const Stmt* loop) {
+        for (size_t s = 0;; ++s) {
+            if (s >= r.summed.size() || loop->bound != r.summed[s] || !enter(loop, &summed)) return nullptr;
+            if (summed.size() == r.summed.size()) return &loop->body;
+            if (loop->body.size() != 1 || loop->body[0]->kind != Stmt::For) return nullptr;
+            loop = loop->body[0];
+        }
+    }
+    // an operand's element at its role's indices, for the output element at `o`
+    bool element(const Expr* e, int buf, bool vec, const std::vector<int>& role, const std::vector<At>& o) const {
+        if (e->kind != (vec ? Expr::VLoad : Expr::Load) || e->id != buf || e->kids.size() != role.size()) return false;
+        for (size_t p = 0; p < role.size(); ++p) {
+            At a;
+            if (!at(e->kids[p], &a)) return false;
+            if (role[p] >= 0 ? !(a == o[role[p]]) : a.var != summed[-1 - role[p]] || a.c != 1) return false;
+        }
+        return true;
+    }
+    static bool add(const Expr* e, bool vec) { return e->kind == (vec ? Expr::VBin : Expr::Bin) && e->op == Op::Add; }
+    static bool zero(const Expr* e) { return e->kind == Expr::Num && e->num == 0 && !std::signbit(e->num); }
+    // the output axes' loops: one variable an axis, every variable of `vars`
+    // used, and (over all of an unrolled axis' offsets) each element once
+    bool axes(const std::vector<At>& o, const std::vector<int>& vars) const {
+        const auto& dims = k.output.dims;
+        if (o.size() != dims.size() || vars.size() != dims.size()) return false;
+        for (size_t d = 0; d < dims.size(); ++d) {
+            if (std::count(vars.begin(), vars.end(), o[d].var) != 1 || o[d].c * bound.at(o[d].var) != dims[d]) return false;
+            for (size_t q = 0; q < d; ++q)
+                if (o[q].var == o[d].var) return false;
+        }
+        return parallel_outer(k) < 0 || (o[0].var == outer[0] && o[0].c == 1);
+    }
+
+    struct Acc {
+        bool vec = false;
+        const Expr *x = nullptr, *w = nullptr, *bias = nullptr;    // the product's operands, the bias
+        bool stored = false;
+        std::vector<At> o;             // where it is stored
     };
-    // elems: the output elements the enclosing output loops cover
-    std::function<void(const std::vector<const Stmt*>&, bool, int64_t, int)> walk = [&](const std::vector<const Stmt*>& body,
-                                                                                       bool inside, int64_t elems, int x) {
-        for (size_t i = 0; ok && i < body.size(); ++i) {
+
+    bool tiled(const std::vector<const Stmt*>& body) {
+        std::map<std::pair<bool, int>, Acc> accs;
+        auto value = [](const Expr* e, bool vec) { return vec ? e->kind == Expr::Splat ? e->kids[0] : nullptr : e; };
+        size_t i = 0;
+        for (; i < body.size() && (body[i]->kind == Stmt::Set || body[i]->kind == Stmt::VSet); ++i) {
+            const bool vec = body[i]->kind == Stmt::VSet;
+            const Expr* v = value(body[i]->value, vec);
+            if (!v || !zero(v) || !accs.emplace(std::make_pair(vec, body[i]->var), Acc{vec}).second) return false;
+        }
+        if (i == body.size() || body[i]->kind != Stmt::For) return false;
+        const auto* products = enter_sum(body[i++]);
+        if (!products) return false;
+        std::map<int, const Expr*> xs;     // scalars holding an element of %0
+        for (auto s : *products) {
+            if (s->kind != Stmt::Set && s->kind != Stmt::VSet) return false;
+            const bool vec = s->kind == Stmt::VSet;
+            const auto acc = accs.find({vec, s->var});
+            if (acc == accs.end()) {
+                if (vec || s->value->kind != Expr::Load) return false;
+                xs[s->var] = s->value;
+                continue;
+            }
+            const Expr* e = s->value;
+            if (!add(e, vec) || e->kids[0]->kind != (vec ? Expr::Vv : Expr::Sv) || e->kids[0]->id != s->var || acc->second.x) return false;
+            const Expr* m = e->kids[1];
+            if (m->kind != (vec ? Expr::VBin : Expr::Bin) || m->op != Op::Mul) return false;
+            const Expr* x = value(m->kids[0], vec);
+            if (!x) return false;
+            // the generic `ein` term (1 * x0) * x1: 1 * x0 is x0 exactly
+            if (x->kind == Expr::Bin && x->op == Op::Mul && x->kids[0]->kind == Expr::Num && x->kids[0]->num == 1) x = x->kids[1];
+            if (x->kind == Expr::Sv) {
+                if (!xs.count(x->id)) return false;
+                x = xs[x->id];
+            }
+            acc->second.x = x;
+            acc->second.w = m->kids[1];
+        }
+        for (int v : summed) bound.erase(v);
+        for (; i < body.size(); ++i) {
             const Stmt* s = body[i];
-            if (s->kind == Stmt::For) {
-                const bool sum = !out_vars.count(s->var);
-                if (sum && !inside && !summed.empty()) ok = false;      // a second chain of sums
-                if (sum) summed.push_back(s->var);
-                walk(s->body, inside || sum, sum ? elems : elems * s->bound, x);
-            } else if (s->kind == Stmt::Set) {
-                const Expr* v = s->value;
-                if (!inside || v->kind != Expr::Load || v->id != 0 || !axes.empty()) { ok = false; break; }
-                for (auto c : v->kids) {
-                    if (c->kind != Expr::Iv) ok = false;
-                    else if (!out_vars.count(c->id)) axes.push_back(c->id);
-                }
-                x = s->var;
-            } else if (s->kind == Stmt::Store) {
-                const Expr* v = s->value;
-                if (s->buf != k.out_buf() || elems != numel) { ok = false; break; }
-                if (!inside && summed.empty()) {
-                    if (v->kind != Expr::Num || v->num != 0 || std::signbit(v->num)) ok = false;
-                    ++zeros;
+            const bool vec = s->kind == Stmt::VSet || s->kind == Stmt::VStore;
+            const Expr* e = s->value;
+            if (s->kind == Stmt::Set || s->kind == Stmt::VSet) {
+                const auto acc = accs.find({vec, s->var});
+                if (acc == accs.end() || k.dtype != Ty::F32 || acc->second.stored || acc->second.bias || !add(e, vec) ||
+                    e->kids[0]->kind != (vec ? Expr::Vv : Expr::Sv) || e->kids[0]->id != s->var)
+                    return false;
+                acc->second.bias = e->kids[1];
+            } else if (s->kind == Stmt::Store || s->kind == Stmt::VStore) {
+                std::vector<At> o;
+                if (s->buf != k.out_buf() || !at(s->index, &o)) return false;
+                if (e->kind == (vec ? Expr::Vv : Expr::Sv)) {
+                    const auto acc = accs.find({vec, e->id});
+                    if (acc == accs.end() || acc->second.stored) return false;
+                    acc->second.stored = true;
+                    acc->second.o = o;
                     continue;
                 }
-                if (v->kind != Expr::Bin || v->op != Op::Add) { ok = false; break; }
-                const Expr *o = v->kids[0], *t = v->kids[1];
-                if (o->kind != Expr::Load || o->id != k.out_buf() || !same(o->kids, s->index)) { ok = false; break; }
-                if (inside) {
-                    if (t->kind != Expr::Bin || t->op != Op::Mul || t->kids[0]->kind != Expr::Sv || t->kids[0]->id != x || x < 0 ||
-                        t->kids[1]->kind != Expr::Load || t->kids[1]->id != 1)
-                        ok = false;
-                    for (auto c : t->kids[1]->kids)
-                        if (c->kind != Expr::Iv) ok = false;
-                    ++terms;
-                } else {
-                    if (t->kind != Expr::Load || t->id != 2 || k.inputs.size() != 3) ok = false;
-                    ++biased;
-                }
+                // the stored element read back, plus the bias
+                std::vector<At> back;
+                if (!add(e, vec) || e->kids[0]->kind != (vec ? Expr::VLoad : Expr::Load) || e->kids[0]->id != k.out_buf() ||
+                    !at(e->kids[0]->kids, &back) || !(back == o))
+                    return false;
+                Acc* to = nullptr;
+                for (auto& a : accs)
+                    if (a.second.vec == vec && a.second.stored && a.second.o == o) to = &a.second;
+                if (!to || to->bias) return false;
+                to->bias = e->kids[1];
             } else {
-                ok = false;
+                return false;
             }
         }
-    };
-    walk(k.body, false, 1, -1);
-    return ok && zeros == 1 && terms == 1 && biased == (k.inputs.size() == 3 ? 1 : 0) && !summed.empty() && axes == summed;
-}
+        // each accumulator's elements are its own, and together they are all
+        const int last = (int)k.output.dims.size() - 1;
+        auto carries = [&](const std::vector<int>& role) { return std::count(role.begin(), role.end(), last) > 0; };
+        std::set<std::vector<int64_t>> seen;
+        int64_t tile = 1;
+        for (const auto& entry : accs) {
+            const Acc& a = entry.second;
+            if (!a.stored || !a.x || (a.bias != nullptr) != (k.inputs.size() == 3) || !axes(a.o, outer)) return false;
+            const auto& first = accs.begin()->second.o;
+            std::vector<int64_t> t;
+            tile = 1;
+            for (size_t d = 0; d < a.o.size(); ++d) {
+                if (a.o[d].var != first[d].var || a.o[d].c != first[d].c) return false;
+                t.push_back(a.o[d].t);
+                if (a.o[d].c > 4096 || (tile *= a.o[d].c) > 4096) return false;
+            }
+            for (int l = 0; l < (a.vec ? k.lanes : 1); ++l, ++t[last])
+                if (t[last] >= a.o[last].c || !seen.insert(t).second) return false;
+            // (a vector runs along its buffer's last axis)
+            if ((a.vec && carries(r.x)) || !element(a.x, 0, false, r.x, a.o)) return false;
+            if ((a.vec && (r.w.empty() || r.w.back() != last)) || !element(a.w, 1, a.vec, r.w, a.o)) return false;
+            if (a.bias) {
+                const bool run = a.vec && carries(r.bias);
+                if (run && r.bias.back() != last) return false;
+                const Expr* b = a.vec && !run ? value(a.bias, true) : a.bias;
+                if (!b || !element(b, 2, run, r.bias, a.o)) return false;
+            }
+        }
+        return !seen.empty() && (int64_t)seen.size() == tile;
+    }
+
+    // the column loops from `loop` in around one store: where it stores (its
+    // loops closed again)
+    const Stmt* row_store(const Stmt* loop, std::vector<At>* o) {
+        std::vector<int> vars = outer;
+        const Stmt* s = loop;
+        while (s->kind == Stmt::For) {
+            if (s->body.size() != 1 || !enter(s, &vars)) return nullptr;
+            s = s->body[0];
+        }
+        if (s->kind != Stmt::Store || s->buf != k.out_buf() || !at(s->index, o) || !axes(*o, vars)) return nullptr;
+        for (size_t v = outer.size(); v < vars.size(); ++v) bound.erase(vars[v]);
+        for (const At& a : *o)
+            if (a.c != 1) return nullptr;
+        return s;
+    }
+    // the axes that the row's own loops index are the same in `o` and `p`
+    bool same_row(const std::vector<At>& o, const std::vector<At>& p) const {
+        for (size_t d = 0; d < o.size(); ++d)
+            for (int v : outer)
+                if ((o[d].var == v) != (p[d].var == v)) return false;
+        return true;
+    }
+    bool adds_to(const Stmt* s, const std::vector<At>& o) const {
+        std::vector<At> back;
+        return add(s->value, false) && s->value->kids[0]->kind == Expr::Load && s->value->kids[0]->id == k.out_buf() &&
+               at(s->value->kids[0]->kids, &back) && back == o;
+    }
+
+    bool row_wise(const std::vector<const Stmt*>& body) {
+        const size_t parts = k.inputs.size();            // zero, sum, and the bias
+        if (k.dtype != Ty::F32 || body.size() != parts) return false;
+        for (auto s : body)
+            if (s->kind != Stmt::For) return false;
+        std::vector<At> row, o;
+        const Stmt* s = row_store(body[0], &row);
+        if (!s || !zero(s->value)) return false;
+        const auto* products = enter_sum(body[1]);
+        if (!products || products->size() != 2 || (*products)[0]->kind != Stmt::Set || (*products)[1]->kind != Stmt::For) return false;
+        const Stmt* x = (*products)[0];
+        s = row_store((*products)[1], &o);
+        if (!s || !same_row(row, o) || !adds_to(s, o)) return false;
+        const Expr* m = s->value->kids[1];
+        if (m->kind != Expr::Bin || m->op != Op::Mul || m->kids[0]->kind != Expr::Sv || m->kids[0]->id != x->var ||
+            !element(x->value, 0, false, r.x, o) || !element(m->kids[1], 1, false, r.w, o))
+            return false;
+        // (%0's element is read outside the column loops)
+        for (int d : r.x)
+            if (d >= 0 && !std::count(outer.begin(), outer.end(), o[d].var)) return false;
+        for (int v : summed) bound.erase(v);
+        if (parts < 3) return true;
+        s = row_store(body[2], &o);
+        return s && same_row(row, o) && adds_to(s, o) && element(s->value->kids[1], 2, false, r.bias, o);
+    }
+};
 
 // ---- the contraction class ---------------------------------------------------------
 struct GemmPlan : ClassPlan {
@@ -916,6 +994,15 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
     long long scale_axis = -1;
     std::vector<long long> batch_scales;
     const auto ws = ty_quant(w.ty) ? w.scale_strides() : std::vector<int64_t>();
+    SumRoles roles;
+    const int rank = (int)o.dims.size();
+    if (is_dot || is_l) {
+        // %0's leading axes are the output's
+        for (int d = 0; d + 1 < rank; ++d) roles.x.push_back(d);
+        roles.x.push_back(-1);
+        roles.w = is_dot ? std::vector<int>{-1, rank - 1} : std::vector<int>{rank - 1, -1};
+        roles.summed = {x.dims.empty() ? 0 : x.dims.back()};
+    }
     if (is_dot) {
         // x[outer..., I, K] . w[K, J] -> [outer..., I, J]   (Contraction::of, lower.rs:700-711)
         if (w.dims.size() != 2 || x.dims.size() < 2 || x.dims.back() != w.dims[0]) return nullptr;
@@ -945,6 +1032,11 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         g.N = w.dims.back();
         g.K = prod(x.dims, 0, x.dims.size() - 1);
         if (o.dims.size() != 2 || o.dims[0] != g.M || o.dims[1] != g.N) return nullptr;
+        roles.summed.assign(x.dims.begin(), x.dims.end() - 1);
+        for (size_t i = 0; i < roles.summed.size(); ++i) roles.x.push_back(-1 - (int)i);
+        roles.w = roles.x;
+        roles.x.push_back(0);
+        roles.w.push_back(1);
         g.sa_m = 1; g.sa_k = g.M; g.sb_k = g.N; g.sb_n = 1; g.sc_m = g.N;
         p->rows_per_iter = 1;
     } else {
@@ -982,6 +1074,10 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         for (int v : v1)
             if (pos(vo, v) < 0 && pos(v0, v) < 0) return nullptr;
         if (summed.empty()) return nullptr;
+        auto role = [&](int v) { return pos(vo, v) >= 0 ? pos(vo, v) : -1 - pos(summed, v); };
+        for (int v : v0) roles.x.push_back(role(v));
+        for (int v : v1) roles.w.push_back(role(v));
+        for (int v : summed) roles.summed.push_back(x.dims[pos(v0, v)]);
         // the loops' nesting depth: the summed axes outermost first
         std::map<int, int> depth;
         std::function<void(const std::vector<const Stmt*>&, int)> walk = [&](const std::vector<const Stmt*>& body, int d) {
@@ -1093,6 +1189,7 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         std::vector<int> m;
         const BufSpec& b = k.inputs[2];
         if (!align(b, o, &m)) return nullptr;
+        roles.bias = m;
         // supported broadcasts: the bias over the last axis (J), over every axis, or a scalar
         const size_t r = o.dims.size();
         if (m.empty()) {
@@ -1117,7 +1214,7 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
         const long long lim = 1ll << 22;   // 32-bit offsets inside a tile
         if (wide || g.sa_m >= lim || g.sa_k >= lim || g.sb_k >= lim || g.sb_n >= lim ||
             (double)g.M * g.N * g.batch * g.K < 8388608.0 || g.M < 32 || g.N < 32 ||
-            !(sequential_sum(k) || row_wise_sum(k)))
+            !OrderedSum(k, roles).holds())
             return nullptr;
         p->seq = true;
         g.splits = 1;
@@ -1141,6 +1238,8 @@ std::unique_ptr<ClassPlan> classify_gemm(const Kernel& k, bool seq) {
                                                      : p->rows_per_iter > 0 && g.M == n0 * p->rows_per_iter)
             p->split = n0;
     }
+    // (a printed nest runs any range of its split loop)
+    if (seq && n0 > 0 && p->split != n0) return nullptr;
     return p;
 }
 

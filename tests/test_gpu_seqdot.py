@@ -96,3 +96,96 @@ def test_rule():
     assert "= 0\n" in row_wise.text and kind(row_wise) == "seqdot"
     narrow = row_wise.text.replace(": f32[", ": bf16[")
     assert kind(row_wise, "bf16", narrow) == "generic"
+
+
+def edits():
+    """(name, text, lanes, type) of nests under a contraction's name that do
+    not compute it, or not in its loops: one edit each of what the lowering
+    writes, at equal sizes wherever that lets the edit stay in bounds."""
+    n = 512
+
+    def each(title, low, dt, changes):
+        for what, *pairs in changes:
+            text = low.text
+            for old, new in pairs:
+                assert old in text, (title, what, old, text)
+                text = text.replace(old, new)
+            assert text != low.text
+            yield f"{title}: {what}", text, low.lanes, dt
+    sum_loop, rows, columns = "for i2 in 0..512", "for i0 in 0..512", "for i1 in 0..512"
+    yield from each("dot_vjp_l", L.dot_vjp_l([O(A(("batch", n), n)), O(A(n, n))], "f32"), "f32", [
+        ("half the sum", (sum_loop, "for i2 in 0..256")),
+        ("half the rows", (rows, "for i0 in 0..256")),
+        ("half the columns", (columns, "for i1 in 0..256")),
+        ("one row of %0", ("%0[i0, i2]", "%0[0, i2]")),
+        ("one row of %1", ("%1[i1, i2]", "%1[0, i2]")),
+        ("one k of %1", ("%1[i1, i2]", "%1[i1, 0]")),
+        ("rows exchanged", ("%0[i0, i2]", "%0[i1, i2]"), ("%1[i1, i2]", "%1[i0, i2]")),
+        ("%0 transposed", ("%0[i0, i2]", "%0[i2, i0]")),
+        ("%1 transposed", ("%1[i1, i2]", "%1[i2, i1]")),
+        ("the diagonal of %0", ("%0[i0, i2]", "%0[i0, i0]")),
+        ("store transposed", ("%2[i0, i1]", "%2[i1, i0]")),
+        ("store of a row's first", ("%2[i0, i1]", "%2[i0, 0]")),
+        ("zero above the columns", ("      s0 = 0\n", ""), ("    for i1 in", "    s0 = 0\n    for i1 in")),
+        ("from one", ("s0 = 0\n", "s0 = 1\n")),
+        # (columns outermost: a partial range of the split loop is of columns)
+        ("loops exchanged", (rows, "for iX in 0..512"), (columns, rows), ("for iX in", "for i1 in")),
+    ])
+    x, w = O(A(("batch", n), n)), O(A(n, n))
+    yield from each("dot", L.dot([x, w], "f32"), "f32", [
+        ("stores exchanged", ("<v= v0", "<v= vX"), ("<v= v1", "<v= v0"), ("<v= vX", "<v= v1")),
+        ("one sum stored twice", ("<v= v1", "<v= v0")),
+        ("one column run stored twice", ("%2[i0, ((i1 * 8) + 4)]", "%2[i0, ((i1 * 8) + 0)]")),
+        ("columns of %1 exchanged", ("((i1 * 8) + 0)]<v>", "((i1 * 8) + X)]<v>"), ("((i1 * 8) + 4)]<v>", "((i1 * 8) + 0)]<v>"),
+         ("((i1 * 8) + X)]<v>", "((i1 * 8) + 4)]<v>")),
+        ("half the columns", ("for i1 in 0..64", "for i1 in 0..32")),
+        ("overlapping columns", ("(i1 * 8)", "(i1 * 4)")),
+        ("one sum twice", ("        s0 = %0[i0, i2]\n        v0", "        s0 = %0[i0, i2]\n        v1 = (v1 + (splat(s0) * %1[i2, ((i1 * 8) + 4)]<v>)<v>)<v>\n        v0")),
+        ("one sum not zeroed", ("      v1 = splat(0)\n", "")),
+        ("half the sum", (sum_loop, "for i2 in 0..256")),
+        ("one k of %0", ("%0[i0, i2]", "%0[i0, 0]")),
+    ])
+    b = O(A(n))
+    yield from each("dot+add f32", L.dot([x, w, b], "f32", epilogue=(True, A(("batch", n), n))), "f32", [
+        ("first biases", ("%2[((i1 * 8) + 0)]", "%2[0]"), ("%2[((i1 * 8) + 4)]", "%2[4]")),
+        ("a row's bias", ("%2[((i1 * 8) + 0)]<v>", "splat(%2[i0])")),
+        ("biases exchanged", ("%2[((i1 * 8) + 0)]", "%2[((i1 * 8) + X)]"), ("%2[((i1 * 8) + 4)]", "%2[((i1 * 8) + 0)]"),
+         ("%2[((i1 * 8) + X)]", "%2[((i1 * 8) + 4)]")),
+        ("one bias twice", ("v1 = (v1 + %2[((i1 * 8) + 4)]<v>)<v>", "v0 = (v0 + %2[((i1 * 8) + 4)]<v>)<v>")),
+    ])
+    yield from each("dot+add bf16", L.dot([x, w, b], "bf16", epilogue=(True, A(("batch", n), n))), "bf16", [
+        ("a bias elsewhere", ("%2[((i1 * 8) + 3)]", "%2[((i1 * 8) + 2)]")),
+        ("a bias twice", ("%3[i0, ((i1 * 8) + 3)] = (%3[i0, ((i1 * 8) + 3)] + %2[((i1 * 8) + 3)])",
+                          "%3[i0, ((i1 * 8) + 2)] = (%3[i0, ((i1 * 8) + 2)] + %2[((i1 * 8) + 2)])")),
+        ("a column left", ("%3[i0, ((i1 * 8) + 3)] = s3", "%3[i0, ((i1 * 8) + 2)] = s3")),
+    ])
+    m, j, k = 1030, 65, 130
+    low = L.dot([O(A(("batch", m), k)), O(A(k, j)), O(A(j))], "f32", epilogue=(True, A(("batch", m), j)))
+    zero = "    for i2 in 0..65 {\n      %3[i0, i2] = 0\n    }\n"
+    yield from each("row-wise", low, "f32", [
+        ("half the sum", ("for i1 in 0..130", "for i1 in 0..65")),
+        ("half the rows", ("for i0 in 0..1030", "for i0 in 0..515")),
+        ("half zeroed", ("for i2 in 0..65 {\n      %3[i0, i2] = 0", "for i2 in 0..32 {\n      %3[i0, i2] = 0")),
+        ("one row zeroed", ("%3[i0, i2] = 0", "%3[0, i2] = 0")),
+        ("one k of %0", ("%0[i0, i1]", "%0[i0, 0]")),
+        ("%0 by column", ("%0[i0, i1]", "%0[i1, i1]")),
+        ("one k of %1", ("%1[i1, i2]", "%1[0, i2]")),
+        ("one bias", ("%2[i2]", "%2[0]")),
+        ("one column twice", ("(%3[i0, i2] + (s0", "(%3[i0, 0] + (s0")),
+        ("zeroed after", (zero, "    }\n"), ("  for i0 in 0..1030 {\n    }\n", "  for i0 in 0..1030 {\n"),
+         ("    for i2 in 0..65 {\n      %3[i0, i2] = (%3[i0, i2] + %2", zero + "    for i2 in 0..65 {\n      %3[i0, i2] = (%3[i0, i2] + %2")),
+    ])
+    q, kk = O(A(("heads", 2), ("seq", n), ("hd", n))), O(A(("heads", 2), ("seq2", n), ("hd", n)))
+    yield from each("ein", L.ein([q, kk], [["heads", "seq", "hd"], ["heads", "seq2", "hd"]], ["heads", "seq", "seq2"], "f32"), "f32", [
+        ("half the sum", ("for i3 in 0..512", "for i3 in 0..256")),
+        ("half the rows", ("for i1 in 0..512", "for i1 in 0..256")),
+        ("half the columns", ("for i2 in 0..512", "for i2 in 0..256")),
+        ("one batch entry", ("for i0 in 0..2", "for i0 in 0..1")),
+    ])
+
+
+def test_edited_nests_keep_their_own_loops():
+    """A nest is taken for what it computes and not for its name: each of
+    these runs as printed."""
+    taken = [name for name, text, lanes, dt in edits() if hip.Compiled(text, dt, lanes, hip.EXACT).kind != "generic"]
+    assert not taken, taken
