@@ -46,6 +46,15 @@ __device__ __forceinline__ unsigned pk_bf16(float a, float b) {
     const f32x2 v = {a, b};
     return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
 }
+// An f32 element is split times 2^16 (exact): bf16 has f32's exponents but not
+// its subnormals' steps (2^-133 against 2^-149), so the parts of an element
+// below 2^-110 would be cut, and one below 2^-134 lost.  Times 2^16 every f32,
+// subnormal ones too, is the sum of its three parts.  Sums leave times 2^-16
+// an operand.  What this pushes past f32's range instead -- an element from
+// 2^112, a sum from 2^96 -- is not finite and is summed again by the f32 MFMAs
+// as any such sum is.
+constexpr float kSplitUp = 65536.f, kSplitDown = 1.f / 65536.f;
+
 template <int ST>
 __device__ __forceinline__ unsigned pk_half(float a, float b) {
     if (ST != kF16) return pk_bf16(a, b);
@@ -182,7 +191,8 @@ struct StageLoader {
         const int some = EDGE && KC && left < BK ? left - k_of(q) : V;
         if constexpr (OP == kOpF32) {
             f32x4 x = __builtin_bit_cast(f32x4, r[q]);
-            if (none) x = f32x4{};
+#pragma unroll
+            for (int e = 0; e < V; ++e) x[e] = none ? 0.f : x[e] * kSplitUp;
             if (EDGE && KC && left < BK) {
 #pragma unroll
                 for (int e = 1; e < V; ++e) x[e] = e < some ? x[e] : 0.f;
@@ -463,10 +473,12 @@ __global__ void __launch_bounds__(64 * NW, 2) staged_gemm_kernel(GemmArgs g) {
     }
     if (kt < nk) block(kt, no, no, 0, 0);
 
-    // The sums, an integer weight's scaled.  Where operands were split or
-    // unscaled, an infinite or NaN sum (an infinite or NaN operand, whose
-    // split is NaN, or a sum past f32's range) is taken again by f32 MFMAs
-    // over the same k of the elements themselves.
+    // The sums: split operands' back at their scale, an integer weight's
+    // times its scale (before, so that only the result can be subnormal).
+    // Where operands were split or unscaled, an infinite or NaN sum (an
+    // infinite or NaN operand, whose split is NaN, or a sum past f32's range
+    // here) is taken again by f32 MFMAs over the same k of the elements
+    // themselves.
     if constexpr (PA == 3 || QUANT) {
         const float* const scales = QUANT ? g.scales + s_off : nullptr;
 #pragma unroll
@@ -480,6 +492,11 @@ __global__ void __launch_bounds__(64 * NW, 2) staged_gemm_kernel(GemmArgs g) {
                         const int n = n0 + wn + j * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
                         v[e] = v[e] * scales[(n < N ? n : N - 1) * g.ss_n];
                     }
+                }
+                if constexpr (PA == 3) {
+                    constexpr float down = PB == 3 ? kSplitDown * kSplitDown : kSplitDown;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) v[e] = v[e] * down;
                 }
                 bool bad = false;
 #pragma unroll

@@ -105,6 +105,65 @@ def test_infinities_and_nans_as_the_f32_tiles_give_them(kind, m, n, k, monkeypat
     assert np.count_nonzero(~fin) > 0 and np.allclose(got[fin], want[fin], rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,m,n,k", [("nn", 256, 384, 512), ("tn", 130, 131, 2050), ("nt", 200, 130, 513)])
+@pytest.mark.parametrize("size", [1e-30, 1e-33, 1e-35, 1e-37, 1e-39, 1e-42])
+@pytest.mark.parametrize("small", [0, 1])
+@pytest.mark.parametrize("up", [False, True])
+def test_small_operands_keep_their_bits(kind, m, n, k, size, small, up):
+    """One operand down to f32's subnormals, whose steps bf16 has not, the
+    other near one or scaled up to give results near one: the band of the
+    sizes above, and for results that are themselves subnormal the rounding
+    of each split's sum and of their total to steps of 2^-149."""
+    hip.init(0)
+    print(f"[split3] {kind} {m}x{n}x{k} at {size} {small} {up}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    v = operands(kind, m, n, k, 1, rng)
+    v[small] = (v[small] * size).astype(np.float32)
+    if up:
+        v[1 - small] = (v[1 - small] * min(1 / size, 1e37)).astype(np.float32)
+    got, c = run(nest(kind, m, n, k), v)
+    want, S = f64(kind, v)
+    splits = int(c.order.split("-split")[1]) if "-split" in c.order else 1
+    gamma = k * 2.0 ** -24 / (1 - k * 2.0 ** -24)
+    bound = 2 * gamma * S + 2.0 ** -23 * (S + np.abs(want)) + (splits + 1) * 2.0 ** -149
+    err = np.abs(got.astype(np.float64).reshape(want.shape) - want)
+    assert np.all(err <= bound), f"{np.count_nonzero(~(err <= bound))} outputs outside the band, {np.max(err / bound):.3g} of it"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("size", [1e-33, 1e-37, 1e-41])
+@pytest.mark.parametrize("scale", [1.0, 1e30])
+def test_small_activations_of_integer_weights(bits, size, scale):
+    """f32 activations are split the same way; the weights' scales multiply
+    the finished sum (a rounding each, and one of the sum before them)."""
+    from presk_amd import quant as Q
+    hip.init(0)
+    print(f"[split3] int{bits} at {size} scales {scale}", flush=True)
+    m, k, n = 64, 513, 130
+    rng = np.random.default_rng(bits)
+    qt = Q.quantize(rng.standard_normal((k, n)), (k, n), Q.Quant(bits, 0))
+    scales = (qt.scales * scale).astype(np.float32)
+    x = (rng.standard_normal((m, k)) * size).astype(np.float32)
+    low = nest("nn", m, n, k)
+    c = hip.Compiled(Q.mark(low.text, 1, Q.of_quant(qt, (k, n))), "f32", low.lanes, hip.FAST)
+    assert c.order.startswith("mfma-f32x3-k16"), c.order
+    out = hip.DeviceBuffer(4 * m * n)
+    ins = [hip.DeviceBuffer.of(x), hip.DeviceBuffer.of(qt.data), out, hip.DeviceBuffer.of(scales)]
+    c.run([b.ptr for b in ins])
+    hip.sync()
+    got = out.download(np.float32).astype(np.float64).reshape(m, n)
+    w = qt.dequantize().astype(np.float64).reshape(k, n) * scale
+    want, S = x.astype(np.float64) @ w, np.abs(x).astype(np.float64) @ np.abs(w)
+    splits = int(c.order.split("-split")[1]) if "-split" in c.order else 1
+    gamma = k * 2.0 ** -24 / (1 - k * 2.0 ** -24)
+    # (dequantize rounds q s to f32, and the scaled scales are rounded: 2^-23 of S)
+    bound = 2 * gamma * S + 2.0 ** -22 * (S + np.abs(want)) + (splits + 1) * 2.0 ** -149
+    err = np.abs(got - want)
+    assert np.all(err <= bound), f"{np.count_nonzero(~(err <= bound))} outputs outside the band, {np.max(err / bound):.3g} of it"
+
+
 def test_rule():
     """Which products take the split operands: more than 64 rows and columns,
     K from 96 (65 at 128 columns); named tiles, other types and integer
