@@ -8,6 +8,7 @@
 #include <sys/stat.h>
 #include <unistd.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -126,9 +127,11 @@ bool build_code_object(const std::string& src, std::vector<char>* code, std::str
     std::vector<char> data(n);
     hiprtcGetCode(prog, data.data());
     hiprtcDestroyProgram(&prog);
-    // best-effort disk cache, written atomically
+    // best-effort disk cache, written atomically (by each of two threads that
+    // build the same source under a name of its own)
     ::mkdir(dir.c_str(), 0755);
-    std::string tmp = path + ".tmp" + std::to_string(::getpid());
+    static std::atomic<unsigned> serial{0};
+    std::string tmp = path + ".tmp" + std::to_string(::getpid()) + "." + std::to_string(serial++);
     {
         std::ofstream f(tmp, std::ios::binary);
         if (f) f.write(data.data(), (std::streamsize)data.size());
@@ -587,22 +590,44 @@ bool meet(const void* a, int64_t na, const void* b, int64_t nb) {
 int64_t buffer_bytes(const BufSpec& s) { return s.numel() * ty_bytes(s.ty); }
 
 // A printed chain's function, from those its first kernel holds; null when it
-// cannot be had (its kernels are then launched one by one).
+// cannot be had (its kernels are then launched one by one).  Built and loaded
+// outside the lock, so that recordings on other threads do not wait for it;
+// of two threads that load the same chain the first one's is kept.
 hipFunction_t chain_function(const presk_hip_kernel* h, const Generated& g) {
-    std::lock_guard<std::mutex> lock(g_chains_mu);
-    for (const auto& c : h->chains)
-        if (c.src == g.src) return c.fn;
+    // (with the lock held)
+    auto held = [&]() -> hipFunction_t {
+        for (const auto& c : h->chains)
+            if (c.src == g.src) return c.fn;
+        return nullptr;
+    };
+    {
+        std::lock_guard<std::mutex> lock(g_chains_mu);
+        if (hipFunction_t fn = held()) return fn;
+        if (h->chains.size() >= kMaxChains) return nullptr;
+    }
     std::vector<char> code;
     std::string err;
     presk_hip_kernel::Chain c{g.src, nullptr, nullptr};
-    if (h->chains.size() >= kMaxChains || (g.phases[0].bounds[0] + 255) / 256 > 0x7fffffffLL ||
-        !build_code_object(g.src, &code, &err) || hipModuleLoadData(&c.module, code.data()) != hipSuccess)
-        return nullptr;
-    if (hipModuleGetFunction(&c.fn, c.module, g.phases[0].fn.c_str()) != hipSuccess) {
+    if ((g.phases[0].bounds[0] + 255) / 256 > 0x7fffffffLL || !build_code_object(g.src, &code, &err)) return nullptr;
+    hipError_t e = hipModuleLoadData(&c.module, code.data());
+    if (e == hipSuccess) {
+        e = hipModuleGetFunction(&c.fn, c.module, g.phases[0].fn.c_str());
+        if (e == hipSuccess) {
+            std::lock_guard<std::mutex> lock(g_chains_mu);
+            hipFunction_t fn = held();
+            if (!fn && h->chains.size() < kMaxChains) {
+                h->chains.push_back(c);
+                return c.fn;
+            }
+            c.fn = fn;
+        }
         (void)hipModuleUnload(c.module);
+    }
+    // the launches that stand in read the last error: a failed load is not theirs
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         return nullptr;
     }
-    h->chains.push_back(c);
     return c.fn;
 }
 

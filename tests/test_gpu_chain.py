@@ -121,3 +121,46 @@ def test_a_recorded_run_of_elementwise_launches(name, r, c, dt, mode):
         hip.lib().presk_hip_batch_release(b)
     if not special and kept[1].guarded:
         assert want[1], "exp past the largest f16 raises the flag"
+
+
+UNARY = ["neg", "exp", "log", "tanh", "sqrt", "sin", "cos", "abs", "gelu", "gelu_deriv", "relu", "heaviside", "sign", "sigmoid",
+         "pow2", "pow3", "pow4", "pow5", "pow6"]
+
+
+@pytest.mark.gpu
+def test_more_runs_than_a_kernel_keeps():
+    """Every graph begins with the same kernel; those past the sixteenth run
+    that it keeps are launched kernel by kernel, with the same results, and
+    recording an earlier one again finds its run."""
+    hip.init(0)
+    r, c, dt = 1024, 512, "f32"
+    m = A(("batch", r), ("model", c))
+    rng = np.random.default_rng(3)
+    x = np.abs(rng.standard_normal(r * c)).astype(np.float32)
+    bx, b0 = hip.DeviceBuffer.of(x), hip.DeviceBuffer(4 * r * c)
+    first = hip.Compiled(L.unary("abs", [O(m)], dt).text, dt, mode=hip.FAST)
+
+    def table(*bufs):
+        return (ctypes.c_void_p * len(bufs))(*[b.ptr for b in bufs])
+    made = []
+    for op in UNARY + UNARY[:2]:
+        print(f"[chain] abs, {op}", flush=True)
+        k, out = hip.Compiled(L.unary(op, [O(m)], dt).text, dt, mode=hip.FAST), hip.DeviceBuffer(4 * r * c)
+        steps = [(first, table(bx, b0)), (k, table(b0, out))]
+        for q, t in steps:
+            hip.check(hip.lib().presk_hip_run(q.handle, t, 0, max(q.split_bound, 0), None))
+        hip.sync()
+        want = out.download(np.uint32)
+        out.upload(np.full(4 * r * c, 0x5A, np.uint8))
+        b = ctypes.c_void_p()
+        hip.check(hip.lib().presk_hip_batch_create(ctypes.byref(b)))
+        made.append((b, steps, k))
+        for q, t in steps:
+            hip.check(hip.lib().presk_hip_batch_add(b, q.handle, t, 0, max(q.split_bound, 0)))
+        hip.check(hip.lib().presk_hip_batch_graph(b))
+        for _ in range(2):
+            hip.check(hip.lib().presk_hip_batch_run(b, None))
+            hip.sync()
+            assert np.array_equal(out.download(np.uint32), want), op
+    for b, _, _ in made:
+        hip.lib().presk_hip_batch_release(b)
