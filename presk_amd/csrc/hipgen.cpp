@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <functional>
 #include <map>
+#include <cstring>
 #include <set>
 #include <sstream>
 
@@ -946,6 +947,25 @@ bool flat_nest(const Kernel& k, FlatNest* out) {
     return true;
 }
 
+// The name a chain is printed under until chain_source numbers it.
+static const char* const kChainFn = "pk_chain_fn";
+
+std::string chain_name(size_t i) { return "pk_chain_" + std::to_string(i); }
+
+std::string chain_source(const std::vector<std::string>& chains) {
+    std::string src = "#include \"devfmt.hpp\"\n";
+    src += "struct PkArgs { void* buf[" + std::to_string(kMaxBufs) + "]; unsigned* flag; long long lo, hi; };\n";
+    src += "typedef unsigned int pk_u32x4 __attribute__((ext_vector_type(4)));\n";
+    const size_t len = std::strlen(kChainFn);
+    for (size_t i = 0; i < chains.size(); ++i) {
+        std::string one = chains[i];
+        const std::string name = chain_name(i);
+        for (size_t at = 0; (at = one.find(kChainFn, at)) != std::string::npos; at += name.size()) one.replace(at, len, name);
+        src += one;
+    }
+    return src;
+}
+
 bool generate_chain(const std::vector<const Kernel*>& kernels, const std::vector<std::vector<int>>& from, Generated* out,
                     std::vector<std::pair<int, int>>* slots, std::string* err) {
     FlatNest f0;
@@ -1066,12 +1086,9 @@ bool generate_chain(const std::vector<const Kernel*>& kernels, const std::vector
         }
     }
     Phase ph;
-    ph.fn = "pk_chain_" + std::to_string(kernels.size());
+    ph.fn = kChainFn;
     ph.bounds.push_back(f0.numel / f0.vec);
-    std::string src = "#include \"devfmt.hpp\"\n";
-    src += "struct PkArgs { void* buf[" + std::to_string(kMaxBufs) + "]; unsigned* flag; long long lo, hi; };\n";
-    src += "typedef unsigned int pk_u32x4 __attribute__((ext_vector_type(4)));\n";
-    src += "__device__ __forceinline__ void " + ph.fn + "_body(const PkArgs& a" + params + ") {\n";
+    std::string src = "__device__ __forceinline__ void " + ph.fn + "_body(const PkArgs& a" + params + ") {\n";
     src += "    const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;\n";
     src += "    if (t0 >= " + total + ") return;\n    bool ovf = false; (void)ovf;\n" + decl + loads + work;
     if (guarded) src += "    if (ovf) atomicOr(a.flag, 1u);\n";

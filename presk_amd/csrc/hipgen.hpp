@@ -60,9 +60,13 @@ bool flat_nest(const Kernel& k, FlatNest* out);
 // registers, as stored; -1: memory.  Every kernel's output is written.  The
 // pointers are the kernels' buffers in order, inputs then output, without the
 // inputs taken from registers (`slots`: kernel and buffer of each).  FAST mode's
-// exp and erf.
+// exp and erf.  The source is one kernel, for chain_source to put beside others.
 bool generate_chain(const std::vector<const Kernel*>& kernels, const std::vector<std::vector<int>>& from, Generated* out,
                     std::vector<std::pair<int, int>>* slots, std::string* err);
+// The source of several chains' kernels as one module, the i-th under
+// chain_name(i).
+std::string chain_source(const std::vector<std::string>& chains);
+std::string chain_name(size_t i);
 
 // The argument block every printed phase takes (by value).
 struct PhaseArgs {

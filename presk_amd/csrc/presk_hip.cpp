@@ -229,18 +229,19 @@ struct presk_hip_kernel {
     // a class kernel's scratch for presk_hip_run, allocated on first use
     mutable void* work = nullptr;
     int mode = PRESK_HIP_EXACT;
-    // printed chains that begin with this kernel (a recorded batch's graph),
-    // loaded as its own module is and unloaded with it: a graph in flight may
-    // still be running their code when its batch is released
-    struct Chain {
+    // the printed chains of a recorded batch whose first one begins with this
+    // kernel, loaded as its own module is and unloaded with it: a graph in
+    // flight may still be running their code when its batch is released
+    struct Chains {
         std::string src;
         hipModule_t module;
-        hipFunction_t fn;
+        std::vector<hipFunction_t> fns;
     };
-    mutable std::vector<Chain> chains;
+    mutable std::vector<Chains> chains;
 };
 
-// The most chains a kernel keeps; a further one is launched kernel by kernel.
+// The most batches' chains a kernel keeps; a further batch's kernels are
+// launched one by one.
 constexpr size_t kMaxChains = 16;
 std::mutex g_chains_mu;
 
@@ -589,46 +590,47 @@ bool meet(const void* a, int64_t na, const void* b, int64_t nb) {
 
 int64_t buffer_bytes(const BufSpec& s) { return s.numel() * ty_bytes(s.ty); }
 
-// A printed chain's function, from those its first kernel holds; null when it
-// cannot be had (its kernels are then launched one by one).  Built and loaded
-// outside the lock, so that recordings on other threads do not wait for it;
-// of two threads that load the same chain the first one's is kept.
-hipFunction_t chain_function(const presk_hip_kernel* h, const Generated& g) {
+// The functions of a batch's printed chains (one source, `n` of them), from
+// those that the first one's first kernel holds; empty when they cannot be had
+// (their kernels are then launched one by one).  Built and loaded outside the
+// lock, so that recordings on other threads do not wait for it; of two threads
+// that load the same source the first one's is kept.
+std::vector<hipFunction_t> chain_functions(const presk_hip_kernel* h, const std::string& src, size_t n) {
     // (with the lock held)
-    auto held = [&]() -> hipFunction_t {
+    auto held = [&]() {
         for (const auto& c : h->chains)
-            if (c.src == g.src) return c.fn;
-        return nullptr;
+            if (c.src == src) return c.fns;
+        return std::vector<hipFunction_t>();
     };
     {
         std::lock_guard<std::mutex> lock(g_chains_mu);
-        if (hipFunction_t fn = held()) return fn;
-        if (h->chains.size() >= kMaxChains) return nullptr;
+        auto fns = held();
+        if (!fns.empty() || h->chains.size() >= kMaxChains) return fns;
     }
     std::vector<char> code;
     std::string err;
-    presk_hip_kernel::Chain c{g.src, nullptr, nullptr};
-    if ((g.phases[0].bounds[0] + 255) / 256 > 0x7fffffffLL || !build_code_object(g.src, &code, &err)) return nullptr;
+    presk_hip_kernel::Chains c{src, nullptr, std::vector<hipFunction_t>(n, nullptr)};
+    if (!build_code_object(src, &code, &err)) return {};
     hipError_t e = hipModuleLoadData(&c.module, code.data());
     if (e == hipSuccess) {
-        e = hipModuleGetFunction(&c.fn, c.module, g.phases[0].fn.c_str());
+        for (size_t i = 0; i < n && e == hipSuccess; ++i) e = hipModuleGetFunction(&c.fns[i], c.module, chain_name(i).c_str());
         if (e == hipSuccess) {
             std::lock_guard<std::mutex> lock(g_chains_mu);
-            hipFunction_t fn = held();
-            if (!fn && h->chains.size() < kMaxChains) {
+            auto fns = held();
+            if (fns.empty() && h->chains.size() < kMaxChains) {
                 h->chains.push_back(c);
-                return c.fn;
+                return c.fns;
             }
-            c.fn = fn;
+            c.fns = fns;
         }
         (void)hipModuleUnload(c.module);
     }
     // the launches that stand in read the last error: a failed load is not theirs
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
+        return {};
     }
-    return c.fn;
+    return c.fns;
 }
 
 // The batch's launches as the graph takes them: runs of elementwise nests
@@ -643,10 +645,15 @@ hipFunction_t chain_function(const presk_hip_kernel* h, const Generated& g) {
 // one's whole output at its own index, and the bytes it writes meet nothing
 // that the run reads or writes.  FAST only: the compiler may order a product's
 // operands differently in the longer kernel, and the sign of a NaN is that of
-// the first one.
+// the first one.  A batch's chains are one source and one module (a module
+// takes 0.3-0.4 ms to load): recording LayerNorm's four 1.74 ms as modules of
+// their own, 0.65 as one (0.19 without chains), and 558 -> 164 ms the first
+// time, when they are compiled; the course step 5.9 -> 3.2 ms.
 void plan_units(presk_hip_batch& b, bool chains) {
     constexpr size_t kMaxChain = 6;
     b.units.clear();
+    std::vector<std::string> sources;                // the chains', each once
+    std::vector<std::pair<size_t, size_t>> printed;  // (unit, its source)
     const size_t n = b.items.size();
     auto flat = [&](const presk_hip_batch::Item& it, FlatNest* f) {
         if (!it.k || it.k->mode != PRESK_HIP_FAST || it.k->plan || it.k->gen.phases.size() != 1) return false;
@@ -707,8 +714,10 @@ void plan_units(presk_hip_batch& b, bool chains) {
             Generated g;
             std::vector<std::pair<int, int>> where;
             std::string err;
-            if (generate_chain(ks, from, &g, &where, &err) &&
-                (u.fn = chain_function(b.items[i].k, g))) {
+            if (generate_chain(ks, from, &g, &where, &err) && (g.phases[0].bounds[0] + 255) / 256 <= 0x7fffffffLL) {
+                const size_t at = std::find(sources.begin(), sources.end(), g.src) - sources.begin();
+                if (at == sources.size()) sources.push_back(g.src);
+                printed.push_back({b.units.size(), at});
                 u.count = (int)count;
                 u.grid = (unsigned)((g.phases[0].bounds[0] + 255) / 256);
                 for (size_t q = 0; q < where.size(); ++q) u.args.buf[q] = b.items[i + where[q].first].bufs[where[q].second];
@@ -719,6 +728,14 @@ void plan_units(presk_hip_batch& b, bool chains) {
         i += (size_t)u.count;
         b.units.push_back(u);
     }
+    if (printed.empty()) return;
+    const auto fns = chain_functions(b.items[b.units[printed[0].first].first].k, chain_source(sources), sources.size());
+    if (fns.empty()) {
+        b.units.assign(n, presk_hip_batch::Unit());
+        for (size_t i = 0; i < n; ++i) b.units[i].first = (int)i;
+        return;
+    }
+    for (const auto& p : printed) b.units[p.first].fn = fns[p.second];
 }
 
 // The batch's items as the branch planner (branches.hpp) reads them.

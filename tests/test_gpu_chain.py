@@ -43,6 +43,9 @@ def runs(r, c):
         # a later launch writes what an earlier one read, or wrote
         "reused": [two("add", "x", "y", "a"), one("neg", "a", "b"), two("mul", "b", "b", "a"), two("sub", "a", "b", "y2"),
                    one("sqrt", "y2", "b")],
+        # three runs of one graph, the first two the same kernels
+        "thrice": [two("add", "x", "y", "a"), one("neg", "a", "b"), two("add", "y", "x", "c"), one("neg", "c", "d"),
+                   two("mul", "x", "y", "e"), two("sub", "e", "row", "f", row)],
         "long": [one("neg", "x", "a0")] + [two("add", f"a{j}", "y", f"a{j + 1}") for j in range(9)],
     }
 
@@ -54,6 +57,7 @@ def runs(r, c):
     ("columns", 1024, 520, "f32", hip.FAST), ("columns", 1027, 512, "bf16", hip.EXACT), ("columns", 1027, 512, "f16", hip.FAST),
     ("apart", 1027, 512, "bf16", hip.FAST), ("apart", 1024, 520, "f32", hip.EXACT), ("shifted", 1027, 512, "f32", hip.FAST),
     ("shifted", 1100, 512, "bf16", hip.FAST), ("reused", 1027, 512, "f32", hip.FAST), ("reused", 1100, 512, "f16", hip.FAST),
+    ("thrice", 1024, 520, "f32", hip.FAST), ("thrice", 1027, 512, "f16", hip.FAST),
     ("long", 1024, 520, "f32", hip.FAST), ("long", 1027, 512, "bf16", hip.FAST)])
 def test_a_recorded_run_of_elementwise_launches(name, r, c, dt, mode):
     print(f"[chain] {name} {r} x {c} {dt} mode {mode}", flush=True)
