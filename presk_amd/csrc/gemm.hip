@@ -1021,39 +1021,6 @@ __global__ void __launch_bounds__(64 * NW) gemm_kernel(GemmArgs g) {
     }
 }
 
-// The split partial sums added in increasing split order, then the epilogue.
-template <int ST>
-__global__ void __launch_bounds__(256) split_reduce_kernel(GemmArgs g) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= g.M * g.N) return;
-    // M * N < 2^31 (the plan's bound): 32-bit division
-    const unsigned nn = (unsigned)g.N, mq = (unsigned)idx / nn;
-    const long long m = mq, n = (unsigned)idx - mq * nn;
-    // the partials in increasing split order, eight loads in flight
-    const long long mn = g.M * g.N;
-    float s = g.work[idx];
-    int p = 1;
-    for (; p + 8 <= g.splits; p += 8) {
-        float w[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) w[q] = g.work[(long long)(p + q) * mn + idx];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) s = s + w[q];
-    }
-    for (; p < g.splits; ++p) s = s + g.work[(long long)p * mn + idx];
-    bool ovf = false;
-    float b = 0.f;
-    // an e8m15 plan keeps bias_kind but passes no bias here: its own last
-    // kernel adds the bias after narrowing the sum
-    if (g.bias) {
-        if (g.bias_kind == 1) b = load_bias<ST>(g.bias, n);
-        else if (g.bias_kind == 2) b = load_bias<ST>(g.bias, idx);
-        else if (g.bias_kind == 3) b = load_bias<ST>(g.bias, 0);
-    }
-    store_out<ST>(g.C, m * g.sc_m + n, s, g.bias != nullptr, b, ovf);
-    if (ovf && g.flag) atomicOr(g.flag, 1u);
-}
-
 // Products with K of at most two k-blocks (the attention's scores: K 64 or
 // 128 in 16-bit storage, 32 or 64 in f32), both operands k-contiguous: a
 // workgroup keeps its 128-row panel of A in LDS for the whole K and streams
@@ -1283,12 +1250,9 @@ hipError_t launch_typed(const GemmArgs& g, hipStream_t stream) {
     const bool fast = g.a_vec && g.b_vec;
     hipError_t e;
     if (!g.b_bits && !g.staged && stream_fits(g)) return stream_launch<ST>(g, stream);
-    if (g.b_bits || g.staged || (ST == kF32 && g.split3)) {
-        e = g.b_bits ? gemm_quant_launch(g, stream) : g.staged ? gemm_ragged_launch(g, stream) : gemm_split_launch(g, stream);
-        if (e != hipSuccess || g.splits <= 1) return e;
-        split_reduce_kernel<ST><<<(unsigned)((g.M * g.N + 255) / 256), 256, 0, stream>>>(g);
-        return hipGetLastError();
-    }
+    if (g.b_bits) return gemm_quant_launch(g, stream);
+    if (g.staged) return gemm_ragged_launch(g, stream);
+    if (ST == kF32 && g.split3) return gemm_split_launch(g, stream);
     if constexpr (ST == kF32) {
     if (g.bm == 256 || g.eight) {
         // 256 x 128 or 256 x 96 tiles of eight waves (4 x 2 waves of 64 x 64
@@ -1303,9 +1267,7 @@ hipError_t launch_typed(const GemmArgs& g, hipStream_t stream) {
             else if (g.bm == 128 && g.bn == 128) e = launch_shape<ST, 2, 4, false, true, 16, 8, 2>(g, stream);
             else if (g.bm == 128 && g.bn == 96) e = launch_shape<ST, 2, 3, false, true, 16, 8, 2>(g, stream);
             else return hipErrorInvalidValue;
-            if (e != hipSuccess || g.splits <= 1) return e;
-            split_reduce_kernel<ST><<<(unsigned)((g.M * g.N + 255) / 256), 256, 0, stream>>>(g);
-            return hipGetLastError();
+            return e == hipSuccess ? split_reduce<ST>(g, stream) : e;
         }
         GemmArgs h = g;
         h.bm = 128;
@@ -1363,10 +1325,7 @@ hipError_t launch_typed(const GemmArgs& g, hipStream_t stream) {
     } else {
         e = fast ? launch_shape<ST, 4, 4, false>(g, stream) : launch_shape<ST, 4, 4, true>(g, stream);
     }
-    if (e != hipSuccess || g.splits <= 1) return e;
-    const long long n = g.M * g.N;
-    split_reduce_kernel<ST><<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(g);
-    return hipGetLastError();
+    return e == hipSuccess ? split_reduce<ST>(g, stream) : e;
 }
 
 __global__ void __launch_bounds__(256) e8_widen_kernel(const unsigned char* __restrict__ src, float* __restrict__ dst,

@@ -42,8 +42,7 @@ struct GemmArgs {
 
 hipError_t gemm_launch(const GemmArgs& g, hipStream_t stream);
 
-// f32 products as six bf16 products of operands split in three (gemm_split.hip);
-// the split-K partials' reduction is the caller's
+// f32 products as six bf16 products of operands split in three (gemm_split.hip)
 bool gemm_split_fits(const GemmArgs& g);
 hipError_t gemm_split_launch(const GemmArgs& g, hipStream_t stream);
 

@@ -599,7 +599,8 @@ hipError_t staged_launch(const GemmArgs& g0, hipStream_t stream) {
         return hipErrorInvalidValue;
     }
 #undef PRESK_STAGED
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? split_reduce<ST>(g, stream) : e;
 }
 
 // each operand one run of elements along k, or along its rows, at strides

@@ -2,6 +2,8 @@
 // element and the bias element, in each storage type.
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include <type_traits>
 
 #include "devfmt.hpp"
@@ -59,5 +61,54 @@ __device__ __forceinline__ float load_bias(const void* p, long long off) {
     if (ST == kBF16) return pk_bf16_to_f32(((const unsigned short*)p)[off]);
     return pk_f16_to_f32(((const unsigned short*)p)[off]);
 }
+
+namespace {
+
+// The split partial sums added in increasing split order, then the epilogue.
+// Each source has its own: a source's code is loaded whole the first time one
+// of its kernels is, and gemm.hip's is 3 MB (the first recording of a dense
+// layer's reverse mode, whose products gemm_split.hip holds, took 11.2 ms with the
+// partials summed there and takes 5.5).
+template <int ST>
+__global__ void __launch_bounds__(256) split_reduce_kernel(GemmArgs g) {
+    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= g.M * g.N) return;
+    // M * N < 2^31 (the plan's bound): 32-bit division
+    const unsigned nn = (unsigned)g.N, mq = (unsigned)idx / nn;
+    const long long m = mq, n = (unsigned)idx - mq * nn;
+    // the partials in increasing split order, eight loads in flight
+    const long long mn = g.M * g.N;
+    float s = g.work[idx];
+    int p = 1;
+    for (; p + 8 <= g.splits; p += 8) {
+        float w[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) w[q] = g.work[(long long)(p + q) * mn + idx];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s = s + w[q];
+    }
+    for (; p < g.splits; ++p) s = s + g.work[(long long)p * mn + idx];
+    bool ovf = false;
+    float b = 0.f;
+    // an e8m15 plan keeps bias_kind but passes no bias here: its own last
+    // kernel adds the bias after narrowing the sum
+    if (g.bias) {
+        if (g.bias_kind == 1) b = load_bias<ST>(g.bias, n);
+        else if (g.bias_kind == 2) b = load_bias<ST>(g.bias, idx);
+        else if (g.bias_kind == 3) b = load_bias<ST>(g.bias, 0);
+    }
+    store_out<ST>(g.C, m * g.sc_m + n, s, g.bias != nullptr, b, ovf);
+    if (ovf && g.flag) atomicOr(g.flag, 1u);
+}
+
+// (nothing to do where K is not split)
+template <int ST>
+hipError_t split_reduce(const GemmArgs& g, hipStream_t stream) {
+    if (g.splits <= 1) return hipSuccess;
+    split_reduce_kernel<ST><<<(unsigned)((g.M * g.N + 255) / 256), 256, 0, stream>>>(g);
+    return hipGetLastError();
+}
+
+}  // namespace
 
 }  // namespace presk
