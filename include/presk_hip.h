@@ -88,7 +88,10 @@ typedef struct {
  *                                   96/128 on f32 storage, 256 x 128/256 on
  *                                   16-bit) and k splits (1-64, single-entry
  *                                   contractions) in place of the planner's,
- *                                   where they apply;
+ *                                   where they apply; f32 operands and integer
+ *                                   weights then multiply on the f32 MFMAs
+ *                                   ("mfma-f32-k4"), whatever the planner's
+ *                                   order was;
  *   PRESK_HIP_CACHE, PRESK_HIP_DUMP  the generated kernels' code-object cache
  *                                   and a directory to keep their sources in. */
 int presk_hip_init(int device);

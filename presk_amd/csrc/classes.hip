@@ -711,6 +711,15 @@ void plan_staged(GemmArgs& g) {
     }
 }
 
+// Whether the environment names tiles (where malformed, init fails).  The tiles
+// it can name are of f32 or 16-bit operands as they are, so operands split,
+// staged or integer do without their own kernels then.
+bool tiles_named() {
+    TileOverride named;
+    std::string ignored;
+    return tile_override(&named, &ignored) && named.bm != 0;
+}
+
 void plan_tiles(GemmArgs& g, bool widened) {
     g.split3 = g.staged = false;
     g.bm = 128;
@@ -718,13 +727,12 @@ void plan_tiles(GemmArgs& g, bool widened) {
     g.stream = true;
     g.tiles_m = (int)((g.M + gemm_tile_m() - 1) / gemm_tile_m());
     // (operands widened from other types and named tiles keep the f32 MFMAs)
-    TileOverride named;
-    std::string ignored;
-    if (!widened && gemm_split_fits(g) && (!tile_override(&named, &ignored) || named.bm == 0)) {
+    const bool named = tiles_named();
+    if (!widened && !named && gemm_split_fits(g)) {
         plan_split3(g);
         return;
     }
-    if (g.storage != kF32 && gemm_ragged_fits(g) && (!tile_override(&named, &ignored) || named.bm == 0)) {
+    if (g.storage != kF32 && !named && gemm_ragged_fits(g)) {
         // operands whose vectors are not whole (of eight, by their sizes and
         // strides: the pointers are the launch's), or few rows of a long K
         bool whole = (g.a_kcontig ? g.K : g.M) % 8 == 0 && (g.b_kcontig ? g.K : g.N) % 8 == 0 &&
@@ -921,7 +929,7 @@ void plan_tiles(GemmArgs& g, bool widened) {
 bool integer_weights(const Kernel& k, GemmPlan& p, int own, long long scale_axis, const std::vector<long long>& batch_scales) {
     GemmArgs& g = p.g;
     const int b = p.swapped ? 0 : 1;
-    if (own < 0 || k.dtype == Ty::E8M15 || !ty_quant(k.inputs[b].ty) || ty_quant(k.inputs[1 - b].ty)) return false;
+    if (tiles_named() || own < 0 || k.dtype == Ty::E8M15 || !ty_quant(k.inputs[b].ty) || ty_quant(k.inputs[1 - b].ty)) return false;
     if (scale_axis < 0 || (int)batch_scales.size() != g.nbatch || g.M > 2048 || g.N < 32 || !gemm_quant_fits(g)) return false;
     g.b_bits = k.inputs[b].ty == Ty::Q8 ? 8 : 4;
     g.ss_n = scale_axis;

@@ -210,3 +210,15 @@ def test_rule():
         assert order(64, 512, 64, "e8m15", bits).startswith("mfma-f32-k4")
     assert order(8, 4096, 4096, "bf16") == "mfma-k16-split8"
     assert order(1999, 1021, 777, "f16") == "mfma-k16"
+
+
+def test_named_tiles_reach_integer_weights(monkeypatch):
+    """PRESK_HIP_GEMM_TILE puts integer weights on the tiles it names, on the
+    f32 MFMAs that have them, as it does f32 operands."""
+    low = nest("nn", 256, 256, 2048, "bf16")
+    text = Q.mark(low.text, 1, Q.of_quant_dims(8, 0, (2048, 256), (2048, 256)))
+    assert hip.Compiled(text, "bf16", low.lanes, hip.FAST).order.startswith("mfma-k16")
+    monkeypatch.setenv("PRESK_HIP_GEMM_TILE", "128x64/4")
+    assert hip.Compiled(text, "bf16", low.lanes, hip.FAST).order == "mfma-f32-k4-split4"
+    monkeypatch.setenv("PRESK_HIP_GEMM_TILE", "256x96")
+    assert hip.Compiled(text, "bf16", low.lanes, hip.FAST).order == "mfma-f32-k4"
