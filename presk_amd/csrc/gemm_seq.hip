@@ -4,12 +4,13 @@
 // printed nest's bits, computed tile by tile.
 //
 // Bound: two VALU instructions a product (mul, add; binary16's products are
-// exact in f32, so one fma).  256 threads hold a 64 x 64 (32 x 32) tile, 4 x 4
-// (2 x 2) outputs each, and 32-deep blocks of both operands as f32 in LDS; a
-// k's operands are read while the k before is multiplied, the next block's
-// loads are in flight while one is multiplied.  Elements are loaded one by one
-// through general strides, along whichever axis is contiguous, so any size
-// and alignment takes the same path.  Rows and columns past the operands
+// exact in f32, so one fma).  256 threads hold a 64 x 64 (32 x 32, 16 x 16) tile,
+// 4 x 4 (2 x 2, 1) outputs each, and 32-deep blocks of both operands as f32 in
+// LDS; a k's operands are read while the k before is multiplied, the next
+// block's loads are in flight while one is multiplied (16-bit elements widened
+// on their way to LDS: on arrival, each load was waited for, 43 ns a k against
+// 32 in f32).  Elements are loaded one by one through general strides, along
+// whichever axis is contiguous, so any size and alignment takes the same path.  Rows and columns past the operands
 // repeat the last, k past them are zero: a sum from +0 is never -0, so adding
 // +0 changes no bit.
 //
@@ -20,6 +21,8 @@
 // GPT's forward at B 8 x T 256: 9.17 -> 2.24 ms.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gemm_store.hpp"
 
 namespace presk {
@@ -27,10 +30,9 @@ namespace presk {
 namespace {
 
 template <int ST>
-__device__ __forceinline__ float widen(const char* p) {
-    if (ST == kF32) return *(const float*)p;
-    if (ST == kBF16) return pk_bf16_to_f32(*(const unsigned short*)p);
-    return pk_f16_to_f32(*(const unsigned short*)p);
+__device__ __forceinline__ float widen(typename std::conditional<ST == kF32, float, unsigned short>::type x) {
+    if constexpr (ST == kF32) return x;
+    else return ST == kBF16 ? pk_bf16_to_f32(x) : pk_f16_to_f32(x);
 }
 
 // One operand's block (ROWS x BK) as f32 in LDS, [k][ROWS + 4]: KC takes BK k
@@ -44,7 +46,8 @@ struct SeqLoader {
     const char* origin;
     long long step;
     unsigned voff[NV];
-    float r[NV];
+    typedef typename std::conditional<ST == kF32, float, unsigned short>::type S;
+    S r[NV];                     // as stored: widened on arrival they would be waited for there
     __device__ __forceinline__ static int row_of(int q) { return KC ? (q * 256 + threadIdx.x) / BK : (q * 256 + threadIdx.x) % ROWS; }
     __device__ __forceinline__ static int k_of(int q) { return KC ? (q * 256 + threadIdx.x) % BK : (q * 256 + threadIdx.x) / ROWS; }
     __device__ __forceinline__ void init(const void* p, long long base, int rows, long long rs, long long ks, int row0) {
@@ -61,16 +64,16 @@ struct SeqLoader {
     __device__ __forceinline__ void load(int left) {
         if (left >= BK) {
 #pragma unroll
-            for (int q = 0; q < NV; ++q) r[q] = widen<ST>(origin + voff[q]);
+            for (int q = 0; q < NV; ++q) r[q] = *(const S*)(origin + voff[q]);
         } else {
 #pragma unroll
-            for (int q = 0; q < NV; ++q) r[q] = k_of(q) < left ? widen<ST>(origin + voff[q]) : 0.f;
+            for (int q = 0; q < NV; ++q) r[q] = k_of(q) < left ? *(const S*)(origin + voff[q]) : S(0);
         }
         origin += step;
     }
     __device__ __forceinline__ void store(float* tile) const {
 #pragma unroll
-        for (int q = 0; q < NV; ++q) tile[k_of(q) * LD + row_of(q)] = r[q];
+        for (int q = 0; q < NV; ++q) tile[k_of(q) * LD + row_of(q)] = widen<ST>(r[q]);
     }
 };
 
@@ -123,33 +126,43 @@ __global__ void __launch_bounds__(256, 4) seq_gemm_kernel(GemmArgs g) {
     lb.store(smem[0] + BK * LA::LD);
     __syncthreads();
     int cur = 0;
-    for (int k0 = 0; k0 < K; k0 += BK, cur ^= 1) {
-        const bool more = k0 + BK < K;
+    for (int kb = 0; kb < K; kb += BK, cur ^= 1) {
+        const bool more = kb + BK < K;
         if (more) {
-            la.load(K - k0 - BK);
-            lb.load(K - k0 - BK);
+            la.load(K - kb - BK);
+            lb.load(K - kb - BK);
         }
         const float* const as = smem[cur];
         const float* const bs = smem[cur] + BK * LA::LD;
-        // each k's operands are read while the k before is multiplied (left
+        // G k's operands are read while the G before are multiplied (left
         // alone the compiler reads the whole block ahead, 256 registers of
-        // it, and one wave a SIMD remains)
-        float a[2][RM], b[2][RN];
-        take<RM>(as, ty, a[0]);
-        take<RN>(bs, tx, b[0]);
+        // it, and one wave a SIMD remains); a 16 x 16 tile's products of one
+        // k are over long before the next k's operands are there
+        constexpr int G = RM == 1 ? 4 : 1;
+        float a[2][G][RM], b[2][G][RN];
 #pragma unroll
-        for (int k = 0; k < BK; ++k) {
-            if (k + 1 < BK) {
-                take<RM>(as + (k + 1) * LA::LD, ty, a[(k + 1) & 1]);
-                take<RN>(bs + (k + 1) * LB::LD, tx, b[(k + 1) & 1]);
-            }
+        for (int k = 0; k < G; ++k) {
+            take<RM>(as + k * LA::LD, ty, a[0][k]);
+            take<RN>(bs + k * LB::LD, tx, b[0][k]);
+        }
+#pragma unroll
+        for (int k0 = 0; k0 < BK; k0 += G) {
+            const int now = k0 / G & 1;
+#pragma unroll
+            for (int k = 0; k < G; ++k)
+                if (k0 + G < BK) {
+                    take<RM>(as + (k0 + G + k) * LA::LD, ty, a[now ^ 1][k]);
+                    take<RN>(bs + (k0 + G + k) * LB::LD, tx, b[now ^ 1][k]);
+                }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < RM; ++i)
+            for (int k = 0; k < G; ++k)
 #pragma unroll
-                for (int j = 0; j < RN; ++j)
-                    acc[i][j] = ST == kF16 ? __builtin_fmaf(a[k & 1][i], b[k & 1][j], acc[i][j])
-                                           : acc[i][j] + a[k & 1][i] * b[k & 1][j];
+                for (int i = 0; i < RM; ++i)
+#pragma unroll
+                    for (int j = 0; j < RN; ++j)
+                        acc[i][j] = ST == kF16 ? __builtin_fmaf(a[now][k][i], b[now][k][j], acc[i][j])
+                                               : acc[i][j] + a[now][k][i] * b[now][k][j];
             __builtin_amdgcn_sched_barrier(0);
         }
         // the sums belong to this block: without this they are moved past the
@@ -206,6 +219,16 @@ hipError_t launch_st(const GemmArgs& g, hipStream_t stream) {
     // 1024 x 1024: 178 and 204).  Larger tiles gain nothing a product and
     // leave waves too few to cover their latency (128 x 64: 195 us).
     const long long t = ((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
+    // And 16 x 16 where even the 32 x 32 ones leave CUs idle, since a workgroup
+    // is one serial chain over K, bound by latency: against the printed nest,
+    // whose threads hold one output each in such shapes, 32 x 32 tiles took up
+    // to 2.4x as long in 16-bit storage (256 x 128 x 11552, bf16, k-contiguous:
+    // printed 274 us, 32 x 32 651) and 16 x 16 ones take 0.1-1.0x (of 900 shapes
+    // all but two of 4 us, K 56 and 112).  From 192 of the 32 x 32 ones on those
+    // are level or ahead (16 x 16 against them: 128-191 0.83-0.97x, 192-255
+    // 0.95-1.14x).
+    const long long t2 = ((g.M + 31) / 32) * ((g.N + 31) / 32) * g.batch;
+    if (t2 < 192) return launch<ST, 1, 1>(g, stream);
     return t >= 768 ? launch<ST, 4, 4>(g, stream) : launch<ST, 2, 2>(g, stream);
 }
 

@@ -26,6 +26,9 @@ def nests(dt):
     out["dot-odd"] = L.dot([x, O(A(130, 65))], dt)                      # (row-wise in f32)
     out["dot+add-odd"] = L.dot([x, O(A(130, 65)), O(A(65))], dt, epilogue=(True, A(("batch", 1030), 65)))
     out["dot-wide"] = L.dot([O(A(("batch", 2049), 33)), O(A(33, 1536))], dt)   # 64 x 64 tiles
+    out["dot-mid"] = L.dot([O(A(("batch", 1001), 70)), O(A(70, 328))], dt)     # 32 x 32 ones, the others 16 x 16
+    out["dot_vjp_l-mid"] = L.dot_vjp_l([O(A(("batch", 1030), 97)), O(A(193, 97))], dt)
+    out["dot_vjp_r-mid"] = L.dot_vjp_r([O(A(("batch", 65), 385)), O(A(("batch", 65), 545))], dt)
     out["dot_vjp_l"] = L.dot_vjp_l([O(A(("batch", 3), ("seq", 257), 129)), O(A(96, 129))], dt)
     out["dot_vjp_r"] = L.dot_vjp_r([O(A(("batch", 7), ("seq", 150), 95)), O(A(("batch", 7), ("seq", 150), 100))], dt)
     q = O(A(("batch", 2), ("heads", 3), ("seq", 150), ("hd", 64)))
