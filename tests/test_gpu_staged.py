@@ -170,6 +170,16 @@ def test_integer_weights_against_float64(name, dt, bits, m, k, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("name", ["dot", "dot_vjp_l"])
+@pytest.mark.parametrize("m,k,n", [(5, 65, 33), (40, 131, 34), (33, 64, 35), (129, 193, 37), (8, 520, 39), (130, 72, 602)])
+def test_int4_vectors_from_the_middle_of_a_byte(name, dt, m, k, n):
+    """Rows of odd and of even lengths, none a whole vector of eight: vectors
+    that start at either half of a byte, and the operand's last ones."""
+    test_integer_weights_against_float64(name, dt, 4, m, k, n)
+
+
+@pytest.mark.gpu
 def test_integer_weights_of_infinite_and_large_activations():
     """An infinity or a NaN gives what the loads' own products give, and a
     finite sum stays finite where x q alone passes f32's range."""
