@@ -85,6 +85,31 @@ def test_ragged_and_few_rows_equal_the_tiles(kind, dt, scale, m, n, k, monkeypat
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("axes", ["columns", "all", "none"])
+@pytest.mark.parametrize("m,n,k", [(130, 66, 97), (70, 67, 130), (129, 193, 97), (65, 191, 96), (257, 384, 97), (40, 1, 33), (5, 2, 70),
+                                   (129, 3, 65), (64, 6, 77), (33, 132, 600)])
+def test_the_bias_of_the_last_columns(axes, dt, m, n, k):
+    """A bias by columns is read in runs of four that end inside it: columns
+    at the end of a run's, a tile's and the operand's, and fewer than four."""
+    hip.init(0)
+    print(f"[staged] bias {axes} {dt} {m}x{n}x{k}", flush=True)
+    out_axes = A(("batch", m), n)
+    b = {"columns": A(n), "all": out_axes, "none": A()}[axes]
+    low = L.dot([O(A(("batch", m), k)), O(A(k, n)), O(b)], dt, epilogue=(True, out_axes))
+    rng = np.random.default_rng(m + n + k)
+    # small integers: every product and sum is exact, each output's rounding the storage's
+    x, w = rng.integers(-3, 4, (m, k)).astype(np.float32), rng.integers(-2, 3, (k, n)).astype(np.float32)
+    bias = rng.integers(-64, 65, [a.len for a in b] or [1]).astype(np.float32) / 8
+    c = hip.Compiled(low.text, dt, low.lanes, hip.FAST)
+    esz = 4 if dt == "f32" else 2
+    out, _ = call(c, [hip.DeviceBuffer.of(fmt.encode(v, dt)) for v in (x, w, bias)], esz * m * n)
+    got = fmt.decode(out.download(np.float32 if dt == "f32" else np.uint16), dt).reshape(m, n)
+    want = fmt.roundtrip(fmt.roundtrip(x @ w, dt) + bias.reshape(bias.shape if axes != "none" else ()), dt)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [(140, 70, 77), (129, 71, 1021), (66, 131, 97)])
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("kind", ["nn", "nt", "tn", "tt"])
