@@ -628,9 +628,9 @@ void apply_override(GemmArgs& g) {
 // (gemm_split.hip): 128-row tiles of 192 or 128 columns by eight waves (one
 // workgroup a CU), 128 or 64 columns by four (two a CU).  A CU's time over
 // the workgroups it is dealt is modelled as its columns over an efficiency
-// measured at full occupancy -- 192 columns 1 (16384 x 384 x 1536 109 us),
-// 128 by eight waves 0.92 (4096 x 1024 x 1024 51 us), by four 1 in pairs
-// (16384 x 1536 x 384 122 us, where the pair's stores overlap) and 0.77
+// measured at full occupancy, the operands in cache -- 192 columns 1 (16384 x
+// 384 x 1536 109 us), 128 by eight waves 0.92 (4096 x 1024 x 1024 51 us), by
+// four 1 in pairs (16384 x 1536 x 384 129 us, where the pair's stores overlap) and 0.77
 // alone (61 us), 64 columns 0.85 and 0.65 -- the earlier on a tie.  A long K
 // over few tiles is split as the f32 tiles' is: as many ranges as fill one
 // round of the CUs, each of at least four 32-deep blocks, or of twelve from
@@ -696,11 +696,16 @@ void plan_staged(GemmArgs& g) {
         long long s = 512 / t;
         // few rows: eight 64-deep blocks a split, four where that leaves CUs
         // idle (8 x 4096 x 4096 split 8 12.0 us, 16 12.6); 128-row tiles: a
-        // K of 256, or of 1024 from 96 tiles on (1999 x 1021 x 777, 112 of
-        // them: unsplit 13.9 us, 4 ways 28.9; 4096 x 65 x 1021, 64: unsplit
-        // 16.3, 4 ways 12.1; int8 weights from 16, their conversion being
-        // the longer part of a block: 128 x 4096 x 4096, 32 tiles, 4 ways 22.8
-        // us, 16 ways 28.4)
+        // K of 256, or of 1024 from 96 tiles on (K 1021 in f16: 4096 x 65, 32
+        // tiles, unsplit 15.0 us, 4 ways 12.0; 1999 x 400, 112 of 64 columns,
+        // unsplit 12.1, 2 ways 14.6; 1999 x 777, 208, 12.9 and 22.2).  The
+        // line lies between those, not where the two cross: at 48 to 95
+        // tiles and K 1021 the four ways cost (1999 x 640, 80: unsplit 14.3,
+        // 4 ways 25.0), at K 4093 they gain up to 128 (64: unsplit 42.4, 4
+        // ways 25.5, the rule's 8 31.3).  Integer weights from 16, their
+        // conversion being the longer part of a block (int8, 4096 x 4096: 128
+        // rows, 32 tiles, 4 ways 23.4 us, 16 ways 29.6; 1536 columns, 12 tiles,
+        // 16 ways 18.9, 8 17.5; at K 1024 16 tiles take 15.3 unsplit, 13.1 4 ways)
         const long long least = g.bm == 32 ? (t * (nkb / 8) >= 256 ? 8 : 4) : (t < (g.b_bits ? 16 : 96) ? 256 : 1024) / unit;
         if (s > nkb / least) s = nkb / least;
         if (s > 64) s = 64;
@@ -922,10 +927,13 @@ void plan_tiles(GemmArgs& g, bool widened) {
 
 // Whether the nest's integer weights are B, read as integers (gemm_quant.hip):
 // their scales constant along K and at one stride along the columns, A k
-// contiguous in its own storage.  From 32 columns (narrower is a row of a
-// tile), and to 2 048 rows: longer calls keep the widened copies' order
-// "mfma-f32-k4", which their callers rely on, and where the copies are a
-// small part of the work.
+// contiguous in its own storage.  From 32 columns and to 2 048 rows: past
+// those the widened copies' order, "mfma-f32-k4", is held by tests (at 4 096 and
+// 16 384 rows, at 3 and 8 columns).  The lines are not where the two paths
+// cross, the integers being ahead on both sides of each: 4096 x 4096 int8
+// weights take 87 us at 2 048 rows in bf16 and 624 on copies at 2 049 (118 as
+// integers), in f32 213 and 572 (280); 31 columns at 512 rows and K 4096 35 us
+// on copies in bf16, 13 as integers.
 bool integer_weights(const Kernel& k, GemmPlan& p, int own, long long scale_axis, const std::vector<long long>& batch_scales) {
     GemmArgs& g = p.g;
     const int b = p.swapped ? 0 : 1;

@@ -8,8 +8,8 @@
 // three bf16 parts) for f32 ones.  The scale multiplies each finished sum, one
 // rounding where the weights' loads f32(q) s round every term.  The path this
 // replaces wrote f32 copies of both operands and of the output to memory and
-// multiplied on the f32 MFMAs: 512 x 4096 x 11008 in bf16 636 -> 73 us,
-// 8 x 4096 x 4096 87 -> 12.4 us, 512 x 4096 x 4096 in f32 215 -> 60 us.
+// multiplied on the f32 MFMAs: 512 x 4096 x 11008 in bf16 636 -> 74 us,
+// 8 x 4096 x 4096 87 -> 12.4 us, 512 x 4096 x 4096 in f32 215 -> 72 us.
 #include "gemm_stage.hpp"
 
 namespace presk {

@@ -20,14 +20,16 @@
 // load's registers to LDS (6.5 VALU instructions an element, one vector
 // between every few MFMAs); splitting after the LDS reads would repeat it in
 // every wave that shares the operand.  Each vector is loaded again as soon as
-// it has been split, a whole block ahead of its use.  Rates against the f32
-// MFMA tiles (operands larger than the Infinity Cache): 16384 x 384 x 1536
-// 162 -> 109 us, 16384 x 1536 x 384 174 -> 122 us, 16384 x 384 x 384 48 -> 33
-// us, 4096 x 1024 x 1024 68 -> 51 us, the weight gradient [384 x 1536] over K
-// 16384 161 -> 109 us.  Large products run at 190-200 TFLOP/s, which is 1.2
-// PFLOP/s of bf16 MFMAs at the 1.75 GHz that the chip holds under them (MFMA
-// pipes 60 % busy by the counters): the power limit.  Short K is bound by
-// each tile's prologue and stores.
+// it has been split, a whole block ahead of its use.  Against the f32 MFMA
+// tiles, operands in cache: 16384 x 384 x 1536 160 -> 109 us (177 TFLOP/s), 16384
+// x 1536 x 384 178 -> 129 us, the weight gradient [384 x 1536] over K 16384 166
+// -> 116 us, 4096 x 1024 x 1024 68 -> 51 us; over rings of operands larger than
+// the Infinity Cache 160 -> 130, 174 -> 151, 174 -> 139 us and 16384 x 384 x 384
+// 48 -> 41.  The MFMA pipes are busy 55, 44 and 51 % of the cycles of the first
+// three, at the 1.85-1.96 GHz that the chip holds under them (2.2 under the f32
+// MFMAs); LDS reads are free of conflicts.  The rest is the splitting beside
+// them, the waits between blocks, and each tile's prologue and stores, which
+// weigh more the shorter K is; their shares were not told apart.
 #include "gemm_stage.hpp"
 
 namespace presk {

@@ -12,8 +12,8 @@
 // (k past the end is zeroed on the way to LDS), and only one that runs past
 // the operand's last element is read element by element (read so at every
 // row's end, those loads' waits left nothing in flight: 1999 x 1021 x 777 in
-// f16 22.3 us, now 16.5; the f32 gradient [384 x 65] over K 16384 27.2, now
-// 23.7).
+// f16 22.3 us against 16.5; the f32 gradient [384 x 65] over K 16384 27.2
+// against 23.7).
 #pragma once
 
 #include <hip/hip_runtime.h>
