@@ -1,7 +1,7 @@
 """EXACT mode's tiled contractions (gemm_seq.hip): the interpreter's bits.
 
 Each output is its products' running sum in index order, so the device must
-equal the oracle's run of the nest byte for byte -- at the edges of the 32 and
+equal the oracle's run of the nest byte for byte -- at the edges of the 16, 32 and
 64 wide tiles and of the 32-deep k-blocks, in every operand layout and storage
 type, batched, with the bias, with infinities, NaNs and subnormal products.
 Nests whose sums run in another order (a realization's `interleaved` or
