@@ -132,6 +132,28 @@ def test_small_operands_keep_their_bits(kind, m, n, k, size, small, up):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,m,n,k", [("nn", 256, 384, 512), ("tn", 130, 131, 2050), ("bias", 200, 130, 513)])
+@pytest.mark.parametrize("sizes", [(2.0 ** 47, 2.0 ** 47), (2.0 ** 50, 2.0 ** 50), (2.0 ** 110, 1.0), (1.0, 2.0 ** 112), (2.0 ** 123, 2.0 ** -60)])
+def test_large_operands_and_sums(kind, m, n, k, sizes):
+    """Elements on both sides of 2^112 and sums of 2^96, past which the split
+    operands' own sums are not finite and the f32 MFMAs' stand in."""
+    hip.init(0)
+    print(f"[split3] {kind} {m}x{n}x{k} at {sizes}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    v = operands(kind, m, n, k, 1, rng)
+    for i in range(2):
+        v[i] = (v[i] * np.float32(sizes[i])).astype(np.float32)
+    if kind == "bias":
+        v[2] = (v[2] * np.float32(sizes[0] * sizes[1])).astype(np.float32)
+    got, _ = run(nest(kind, m, n, k), v)
+    want, S = f64(kind, v)
+    gamma = k * 2.0 ** -24 / (1 - k * 2.0 ** -24)
+    bound = 2 * gamma * S + 2.0 ** -23 * (S + np.abs(want))
+    err = np.abs(got.astype(np.float64).reshape(want.shape) - want)
+    assert np.all(np.isfinite(got)) and np.all(err <= bound), f"{np.count_nonzero(~(err <= bound))} outputs outside the band"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("size", [1e-33, 1e-37, 1e-41])
 @pytest.mark.parametrize("scale", [1.0, 1e30])
